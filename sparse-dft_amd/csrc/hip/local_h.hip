@@ -5,10 +5,10 @@
 //   A  k_sticks_backward : gather psi into the (x,y) sticks of the G-sphere,
 //                          z-FFT (natural -> slot order), store stick buffer
 //                          T1[column][z slot][stick]  (coalesced over sticks)
-//   B  k_planes          : per (z slot, column) xy-plane in LDS: scatter the
-//                          sticks, y- and x-FFT to slots, x V(r) in slot
-//                          order, x- and y-FFT back to natural order, keep
-//                          only the sticks -> T2
+//   B  k_plane_local     : per (z slot, column) xy-plane in LDS: the sticks,
+//                          y- and x-FFT to slots, x V(r) in slot order, x- and
+//                          y-FFT back to natural order, only the sticks -> T2
+//                          (k_planes where its LDS does not suffice)
 //   C  k_sticks_forward  : z-FFT from slots to natural order, gather onto the
 //                          sphere, add the kinetic term and divide by N
 //
@@ -22,6 +22,7 @@
 #include "fft_dispatch.hpp"
 #include "fft_lengths.hpp"
 #include "local_h.hpp"
+#include "sphere_fft.hpp"
 
 namespace sdft_hip {
 
@@ -355,10 +356,16 @@ hipError_t launch_local_h(const GridPlanDev& p, const double* x, long ldx, long 
   const T* v = reinterpret_cast<const T*>(sizeof(T) == 8 ? (const void*)p.v64 : (const void*)p.v32);
   hipLaunchKernelGGL(k_sticks_backward<T>, ga, dim3(256), lds_lines, stream, x, ldx, p.stick_g, p.nsticks, p.n2, spb,
                      twz, reinterpret_cast<cx<T>*>(t1));
-  const size_t lds_plane = plane_lds_bytes<T>(p.n0, p.n1);
-  launch_k_planes<T>(dim3(p.n2, (unsigned)columns), lds_plane, stream,
-                     reinterpret_cast<const cx<T>*>(t1), reinterpret_cast<cx<T>*>(t2), p.stick_xy, p.nsticks, p.n0,
-                     p.n1, p.n2, twx, twy, v, 0, p.xstart[0], p.xlines[0], p.xstart[1], p.xlines[1]);
+  PlaneLocalPlan plane;
+  if (plan_plane_local<T>(p, plane)) {
+    const hipError_t e = launch_plane_local<T>(p, plane, t1, t2, columns, stream);
+    if (e != hipSuccess) return e;
+  } else {
+    const size_t lds_plane = plane_lds_bytes<T>(p.n0, p.n1);
+    launch_k_planes<T>(dim3(p.n2, (unsigned)columns), lds_plane, stream,
+                       reinterpret_cast<const cx<T>*>(t1), reinterpret_cast<cx<T>*>(t2), p.stick_xy, p.nsticks, p.n0,
+                       p.n1, p.n2, twx, twy, v, 0, p.xstart[0], p.xlines[0], p.xstart[1], p.xlines[1]);
+  }
   hipLaunchKernelGGL(k_sticks_forward<T>, ga, dim3(256), lds_lines, stream, reinterpret_cast<const cx<T>*>(t2),
                      p.stick_g, p.nsticks, p.n2, spb, twz, x, ldx, kinetic, y, ldy, 0.0, double(p.count));
   return hipGetLastError();

@@ -11,6 +11,7 @@ struct GridPlanDev {
   int nsticks = 0;                // distinct (x,y) columns touched by the sphere
   const int* stick_g = nullptr;   // nsticks * n2: sphere index at natural z, or -1
   const int* stick_xy = nullptr;  // nsticks: x*n1 + y
+  const int* stick_map = nullptr;  // n0 * n1: stick of natural (x, y), or -1
   const void* tw64[3] = {nullptr, nullptr, nullptr};  // per axis (cos, sin) FP64
   const void* tw32[3] = {nullptr, nullptr, nullptr};  // per axis FP32
   const double* v64 = nullptr;    // V(r) in slot order [zs][xs][ys]
@@ -18,6 +19,8 @@ struct GridPlanDev {
   // x-lines that hold sticks, as two ranges [start, start + lines) of natural
   // x: the y-transforms of the local H run on these lines only
   int xstart[2] = {0, 0}, xlines[2] = {0, 0};
+  // no stick has y in [ylow, yhigh)
+  int ylow = 0, yhigh = 0;
 };
 
 // y(:,c) = T x(:,c) + FFT_fwd(V . FFT_bwd(x(:,c))) / N for c < columns.

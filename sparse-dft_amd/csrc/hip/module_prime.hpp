@@ -9,6 +9,8 @@
 namespace sdft_hip {
 
 hipError_t prime_module_local_h();
+hipError_t prime_module_plane_local_f64();
+hipError_t prime_module_plane_local_f32();
 hipError_t prime_module_gemm();
 hipError_t prime_module_davidson_kernels();
 hipError_t prime_module_tridiag();

@@ -127,6 +127,20 @@ HostGridPlan build_full_plan(std::array<int, 3> shape) {
 void DeviceGrid::upload(const HostGridPlan& h, hipStream_t s) {
   stick_g.upload(h.stick_g.data(), h.stick_g.size(), s);
   stick_xy.upload(h.stick_xy.data(), h.stick_xy.size(), s);
+  std::vector<int> map(std::size_t(h.shape[0]) * h.shape[1], -1);
+  for (std::size_t i = 0; i < h.stick_xy.size(); ++i) map[std::size_t(h.stick_xy[i])] = int(i);
+  stick_map.upload(map.data(), map.size(), s);
+  // the widest run of y around the middle of the axis without a stick
+  const int n1 = h.shape[1];
+  std::vector<char> seen(std::size_t(n1), 0);
+  for (int key : h.stick_xy) seen[std::size_t(key % n1)] = 1;
+  dev.ylow = dev.yhigh = n1 / 2;
+  if (seen[std::size_t(n1 / 2)]) {
+    dev.ylow = dev.yhigh = n1;
+  } else {
+    while (dev.ylow > 0 && !seen[std::size_t(dev.ylow - 1)]) --dev.ylow;
+    while (dev.yhigh < n1 && !seen[std::size_t(dev.yhigh)]) ++dev.yhigh;
+  }
   dev.n0 = h.shape[0];
   dev.n1 = h.shape[1];
   dev.n2 = h.shape[2];
@@ -135,6 +149,7 @@ void DeviceGrid::upload(const HostGridPlan& h, hipStream_t s) {
   dev.nsticks = h.nsticks();
   dev.stick_g = stick_g.p;
   dev.stick_xy = stick_xy.p;
+  dev.stick_map = stick_map.p;
   for (int r = 0; r < 2; ++r) {
     dev.xstart[r] = h.xstart[r];
     dev.xlines[r] = h.xlines[r];
@@ -173,7 +188,8 @@ void prime_libraries(int device) {
   std::lock_guard<std::mutex> lock(m);
   if (std::find(primed.begin(), primed.end(), device) != primed.end()) return;
   rocblas_initialize();
-  for (hipError_t (*f)() : {prime_module_local_h, prime_module_gemm, prime_module_davidson_kernels,
+  for (hipError_t (*f)() : {prime_module_local_h, prime_module_plane_local_f64,
+                            prime_module_plane_local_f32, prime_module_gemm, prime_module_davidson_kernels,
                             prime_module_tridiag, prime_module_tridiag_eig, prime_module_realspace,
                             prime_module_batch})
     check(f(), "kernel code object");
@@ -705,7 +721,7 @@ void* DeviceOperator::stick_buffer(int which, std::size_t columns, Precision pre
 }
 
 std::size_t DeviceOperator::device_bytes() const {
-  std::size_t b = grid_.stick_g.bytes() + grid_.stick_xy.bytes();
+  std::size_t b = grid_.stick_g.bytes() + grid_.stick_xy.bytes() + grid_.stick_map.bytes();
   for (int a = 0; a < 3; ++a) b += grid_.tw64[a].bytes() + grid_.tw32[a].bytes();
   b += onsite_d_.bytes() + onsite_q_.bytes() + v64_.bytes() + kinetic_d_.bytes() + b64_.bytes() + dblk_.bytes() +
        qblk_.bytes() + v32_.bytes() + b32_.bytes() + atom_offset_.bytes() + atom_rows_.bytes() + block_offset_.bytes() +

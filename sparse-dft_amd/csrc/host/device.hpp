@@ -96,7 +96,7 @@ HostGridPlan build_full_plan(std::array<int, 3> shape);
 // Device copy of a grid plan with twiddles (potential buffers owned separately).
 struct DeviceGrid {
   GridPlanDev dev;
-  DevBuf<int> stick_g, stick_xy;
+  DevBuf<int> stick_g, stick_xy, stick_map;
   DevBuf<double> tw64[3];
   DevBuf<float> tw32[3];
   void upload(const HostGridPlan& h, hipStream_t s);

@@ -26,67 +26,6 @@
 
 namespace sdft_hip {
 
-namespace {
-
-template <typename T>
-__device__ __forceinline__ cx<T> load_cx(const double* p) {
-  const double2 v = *reinterpret_cast<const double2*>(p);
-  return {T(v.x), T(v.y)};
-}
-
-}  // namespace
-
-// Elements of a stick workgroup per thread whose loads are issued together
-// (sticks_per_block keeps a workgroup at <= 2048 elements, 8 per thread of
-// 256): the sphere indices first, then every gather they address, so a thread
-// waits for two memory round trips instead of two per element.
-constexpr int kGatherPer = 8;
-
-// A: grid (ceil(nsticks / spb), columns)
-template <typename T>
-__global__ __launch_bounds__(256) void k_sticks_backward(const double* __restrict__ x, long ldx,
-                                                         const int* __restrict__ stick_g, int nsticks, int n2, int spb,
-                                                         const cx<T>* __restrict__ tw_z, cx<T>* __restrict__ t1) {
-  extern __shared__ unsigned char smem_raw[];
-  cx<T>* lines = reinterpret_cast<cx<T>*>(smem_raw);
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int first = blockIdx.x * spb;
-  const int nl = min(spb, nsticks - first);
-  const long col = blockIdx.y;
-  const double* xc = x + 2 * col * ldx;
-  const int ls = line_stride(n2);
-  const int total = nl * n2;
-  const int* sg = stick_g + (long)first * n2;
-  for (int e0 = 0; e0 < total; e0 += kGatherPer * nt) {
-    int g[kGatherPer];
-#pragma unroll
-    for (int u = 0; u < kGatherPer; ++u) {
-      const int e = e0 + tid + u * nt;
-      g[u] = e < total ? sg[e] : -1;
-    }
-    cx<T> v[kGatherPer];
-#pragma unroll
-    for (int u = 0; u < kGatherPer; ++u) v[u] = g[u] >= 0 ? load_cx<T>(xc + 2L * g[u]) : cx<T>{T(0), T(0)};
-#pragma unroll
-    for (int u = 0; u < kGatherPer; ++u) {
-      const int e = e0 + tid + u * nt;
-      if (e < total) {
-        const int s = e / n2, z = e - s * n2;
-        lines[s * ls + z] = v[u];
-      }
-    }
-  }
-  __syncthreads();
-  LineGeom geom{nl, ls, 1, false};
-  geom.fast_group = true;
-  line_fft_dispatch<T, +1, true>(n2, lines, geom, tw_z, tid, nt);
-  cx<T>* out = t1 + col * (long)n2 * nsticks;
-  for (int e = tid; e < nl * n2; e += nt) {
-    const int zs = e / nl, s = e - zs * nl;
-    out[(long)zs * nsticks + first + s] = lines[s * ls + zs];
-  }
-}
-
 // B: grid (n2 slots, columns). mode 0: local H (bwd, x V, fwd, keep sticks);
 // mode 1: backward only, whole plane stored in slot order (potential setup).
 // In mode 0 the y-transforms run only on the x-lines that hold sticks (the
@@ -193,63 +132,6 @@ void launch_k_planes(dim3 grid, size_t lds, hipStream_t stream, Args... args) {
   }
 }
 
-// C: grid (ceil(nsticks / spb), columns). y = T x + local / N
-template <typename T>
-__global__ __launch_bounds__(256) void k_sticks_forward(const cx<T>* __restrict__ t2, const int* __restrict__ stick_g,
-                                                        int nsticks, int n2, int spb, const cx<T>* __restrict__ tw_z,
-                                                        const double* __restrict__ x, long ldx,
-                                                        const double* __restrict__ kinetic, double* __restrict__ y,
-                                                        long ldy, double inv_count_unused, double count) {
-  extern __shared__ unsigned char smem_raw[];
-  cx<T>* lines = reinterpret_cast<cx<T>*>(smem_raw);
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int first = blockIdx.x * spb;
-  const int nl = min(spb, nsticks - first);
-  const long col = blockIdx.y;
-  const cx<T>* in = t2 + col * (long)n2 * nsticks;
-  const int ls = line_stride(n2);
-  for (int e = tid; e < nl * n2; e += nt) {
-    const int zs = e / nl, s = e - zs * nl;
-    lines[s * ls + zs] = in[(long)zs * nsticks + first + s];
-  }
-  __syncthreads();
-  LineGeom geom{nl, ls, 1, false};
-  geom.fast_group = true;
-  line_fft_dispatch<T, -1, false>(n2, lines, geom, tw_z, tid, nt);
-  const double* xc = x + 2 * col * ldx;
-  double* yc = y + 2 * col * ldy;
-  const int total = nl * n2;
-  const int* sg = stick_g + (long)first * n2;
-  for (int e0 = 0; e0 < total; e0 += kGatherPer * nt) {
-    int g[kGatherPer];
-#pragma unroll
-    for (int u = 0; u < kGatherPer; ++u) {
-      const int e = e0 + tid + u * nt;
-      g[u] = e < total ? sg[e] : -1;
-    }
-    double t[kGatherPer];
-    double2 xi[kGatherPer];
-#pragma unroll
-    for (int u = 0; u < kGatherPer; ++u) {
-      if (g[u] >= 0) {
-        t[u] = kinetic[g[u]];
-        xi[u] = *reinterpret_cast<const double2*>(xc + 2L * g[u]);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kGatherPer; ++u) {
-      if (g[u] < 0) continue;
-      const int e = e0 + tid + u * nt;
-      const int s = e / n2, z = e - s * n2;
-      const cx<T> w = lines[s * ls + z];
-      double2 r;
-      r.x = t[u] * xi[u].x + double(w.x) / count;
-      r.y = t[u] * xi[u].y + double(w.y) / count;
-      *reinterpret_cast<double2*>(yc + 2L * g[u]) = r;
-    }
-  }
-}
-
 // S local part: y = scale * x (used when the operator has no projectors)
 __global__ void k_scale_copy(const double* __restrict__ x, long ldx, double* __restrict__ y, long ldy, long rows,
                              double scale) {
@@ -322,15 +204,6 @@ __global__ void k_potential_to_natural(const double* __restrict__ v64, int n0, i
 }
 
 // ------------------------------------------------------------ host launchers
-namespace {
-int sticks_per_block(int n2) {
-  int spb = 2048 / n2;
-  if (spb < 1) spb = 1;
-  if (spb > 64) spb = 64;
-  return spb;
-}
-}  // namespace
-
 int max_lds_bytes() {
   static int bytes = [] {
     int dev = 0, v = 0;
@@ -347,15 +220,10 @@ hipError_t launch_local_h(const GridPlanDev& p, const double* x, long ldx, long 
   if (columns <= 0) return hipSuccess;
   // one xy-plane per workgroup must fit the LDS of one workgroup
   if (plane_lds_bytes<T>(p.n0, p.n1) > size_t(max_lds_bytes())) return hipErrorInvalidConfiguration;
-  const int spb = sticks_per_block(p.n2);
-  const dim3 ga((p.nsticks + spb - 1) / spb, (unsigned)columns);
-  const size_t lds_lines = size_t(spb) * line_stride(p.n2) * sizeof(cx<T>);
   const cx<T>* twx = reinterpret_cast<const cx<T>*>(sizeof(T) == 8 ? p.tw64[0] : p.tw32[0]);
   const cx<T>* twy = reinterpret_cast<const cx<T>*>(sizeof(T) == 8 ? p.tw64[1] : p.tw32[1]);
-  const cx<T>* twz = reinterpret_cast<const cx<T>*>(sizeof(T) == 8 ? p.tw64[2] : p.tw32[2]);
   const T* v = reinterpret_cast<const T*>(sizeof(T) == 8 ? (const void*)p.v64 : (const void*)p.v32);
-  hipLaunchKernelGGL(k_sticks_backward<T>, ga, dim3(256), lds_lines, stream, x, ldx, p.stick_g, p.nsticks, p.n2, spb,
-                     twz, reinterpret_cast<cx<T>*>(t1));
+  if (const hipError_t e = launch_sticks_backward<T>(p, x, ldx, columns, t1, stream); e != hipSuccess) return e;
   PlaneLocalPlan plane;
   if (plan_plane_local<T>(p, plane)) {
     const hipError_t e = launch_plane_local<T>(p, plane, t1, t2, columns, stream);
@@ -366,9 +234,7 @@ hipError_t launch_local_h(const GridPlanDev& p, const double* x, long ldx, long 
                        reinterpret_cast<const cx<T>*>(t1), reinterpret_cast<cx<T>*>(t2), p.stick_xy, p.nsticks, p.n0,
                        p.n1, p.n2, twx, twy, v, 0, p.xstart[0], p.xlines[0], p.xstart[1], p.xlines[1]);
   }
-  hipLaunchKernelGGL(k_sticks_forward<T>, ga, dim3(256), lds_lines, stream, reinterpret_cast<const cx<T>*>(t2),
-                     p.stick_g, p.nsticks, p.n2, spb, twz, x, ldx, kinetic, y, ldy, 0.0, double(p.count));
-  return hipGetLastError();
+  return launch_sticks_forward<T>(p, t2, columns, x, ldx, kinetic, y, ldy, stream);
 }
 
 template hipError_t launch_local_h<double>(const GridPlanDev&, const double*, long, long, const double*, double*, long,
@@ -399,11 +265,7 @@ hipError_t launch_scale_copy(const double* x, long ldx, double* y, long ldy, lon
 hipError_t launch_potential_setup(const GridPlanDev& full, const double* grid, void* t1, void* t2, double* v64,
                                   float* v32, double* block_ratio, int ratio_blocks, hipStream_t stream) {
   if (plane_lds_bytes<double>(full.n0, full.n1) > size_t(max_lds_bytes())) return hipErrorInvalidConfiguration;
-  const int spb = sticks_per_block(full.n2);
-  const dim3 ga((full.nsticks + spb - 1) / spb, 1);
-  const size_t lds_lines = size_t(spb) * line_stride(full.n2) * sizeof(cx<double>);
-  hipLaunchKernelGGL(k_sticks_backward<double>, ga, dim3(256), lds_lines, stream, grid, 0L, full.stick_g, full.nsticks,
-                     full.n2, spb, reinterpret_cast<const cx<double>*>(full.tw64[2]), reinterpret_cast<cx<double>*>(t1));
+  if (const hipError_t e = launch_sticks_backward<double>(full, grid, 0, 1, t1, stream); e != hipSuccess) return e;
   const size_t lds_plane = plane_lds_bytes<double>(full.n0, full.n1);
   launch_k_planes<double>(dim3(full.n2, 1), lds_plane, stream,
                      reinterpret_cast<const cx<double>*>(t1), reinterpret_cast<cx<double>*>(t2), full.stick_xy,
@@ -469,11 +331,7 @@ hipError_t launch_backward_planes(const GridPlanDev& p, const double* x, long ld
                                   hipStream_t stream) {
   if (columns <= 0) return hipSuccess;
   if (plane_lds_bytes<double>(p.n0, p.n1) > size_t(max_lds_bytes())) return hipErrorInvalidConfiguration;
-  const int spb = sticks_per_block(p.n2);
-  const dim3 ga((p.nsticks + spb - 1) / spb, (unsigned)columns);
-  const size_t lds_lines = size_t(spb) * line_stride(p.n2) * sizeof(cx<double>);
-  hipLaunchKernelGGL(k_sticks_backward<double>, ga, dim3(256), lds_lines, stream, x, ldx, p.stick_g, p.nsticks, p.n2,
-                     spb, reinterpret_cast<const cx<double>*>(p.tw64[2]), reinterpret_cast<cx<double>*>(t1));
+  if (const hipError_t e = launch_sticks_backward<double>(p, x, ldx, columns, t1, stream); e != hipSuccess) return e;
   const size_t lds_plane = plane_lds_bytes<double>(p.n0, p.n1);
   launch_k_planes<double>(dim3(p.n2, (unsigned)columns), lds_plane, stream,
                      reinterpret_cast<const cx<double>*>(t1), reinterpret_cast<cx<double>*>(t2), p.stick_xy,
@@ -488,14 +346,9 @@ hipError_t launch_backward_full(const GridPlanDev& p, const double* x, long ldx,
                                 hipStream_t stream) {
   if (columns <= 0) return hipSuccess;
   if (plane_lds_bytes<T>(p.n0, p.n1) > size_t(max_lds_bytes())) return hipErrorInvalidConfiguration;
-  const int spb = sticks_per_block(p.n2);
-  const dim3 ga((p.nsticks + spb - 1) / spb, (unsigned)columns);
-  const size_t lds_lines = size_t(spb) * line_stride(p.n2) * sizeof(cx<T>);
   const cx<T>* twx = reinterpret_cast<const cx<T>*>(sizeof(T) == 8 ? p.tw64[0] : p.tw32[0]);
   const cx<T>* twy = reinterpret_cast<const cx<T>*>(sizeof(T) == 8 ? p.tw64[1] : p.tw32[1]);
-  const cx<T>* twz = reinterpret_cast<const cx<T>*>(sizeof(T) == 8 ? p.tw64[2] : p.tw32[2]);
-  hipLaunchKernelGGL(k_sticks_backward<T>, ga, dim3(256), lds_lines, stream, x, ldx, p.stick_g, p.nsticks, p.n2, spb,
-                     twz, reinterpret_cast<cx<T>*>(t1));
+  if (const hipError_t e = launch_sticks_backward<T>(p, x, ldx, columns, t1, stream); e != hipSuccess) return e;
   const size_t lds_plane = plane_lds_bytes<T>(p.n0, p.n1);
   launch_k_planes<T>(dim3(p.n2, (unsigned)columns), lds_plane, stream,
                      reinterpret_cast<const cx<T>*>(t1), reinterpret_cast<cx<T>*>(t2), p.stick_xy, p.nsticks, p.n0,
@@ -510,18 +363,12 @@ hipError_t launch_forward_planes(const GridPlanDev& p, const void* planes, long 
   if (plane_lds_bytes<T>(p.n0, p.n1) > size_t(max_lds_bytes())) return hipErrorInvalidConfiguration;
   const cx<T>* twx = reinterpret_cast<const cx<T>*>(sizeof(T) == 8 ? p.tw64[0] : p.tw32[0]);
   const cx<T>* twy = reinterpret_cast<const cx<T>*>(sizeof(T) == 8 ? p.tw64[1] : p.tw32[1]);
-  const cx<T>* twz = reinterpret_cast<const cx<T>*>(sizeof(T) == 8 ? p.tw64[2] : p.tw32[2]);
   const size_t lds_plane = plane_lds_bytes<T>(p.n0, p.n1);
   launch_k_planes<T>(dim3(p.n2, (unsigned)columns), lds_plane, stream,
                      reinterpret_cast<const cx<T>*>(planes), reinterpret_cast<cx<T>*>(t_sticks), p.stick_xy,
                      p.nsticks, p.n0, p.n1, p.n2, twx, twy, (const T*)nullptr, 2, p.xstart[0], p.xlines[0],
                      p.xstart[1], p.xlines[1]);
-  const int spb = sticks_per_block(p.n2);
-  const dim3 ga((p.nsticks + spb - 1) / spb, (unsigned)columns);
-  const size_t lds_lines = size_t(spb) * line_stride(p.n2) * sizeof(cx<T>);
-  hipLaunchKernelGGL(k_sticks_forward<T>, ga, dim3(256), lds_lines, stream, reinterpret_cast<const cx<T>*>(t_sticks),
-                     p.stick_g, p.nsticks, p.n2, spb, twz, x, ldx, diag, y, ldy, 0.0, double(p.count));
-  return hipGetLastError();
+  return launch_sticks_forward<T>(p, t_sticks, columns, x, ldx, diag, y, ldy, stream);
 }
 
 template hipError_t launch_backward_full<double>(const GridPlanDev&, const double*, long, long, void*, void*,
@@ -572,7 +419,7 @@ hipError_t launch_potential_to_natural(const GridPlanDev& p, const double* v64, 
 // Loads this file's code object on the calling thread (see module_prime.hpp).
 hipError_t prime_module_local_h() {
   hipFuncAttributes a{};
-  return hipFuncGetAttributes(&a, reinterpret_cast<const void*>(k_sticks_backward<double>));
+  return hipFuncGetAttributes(&a, reinterpret_cast<const void*>(k_planes<double, 1024>));
 }
 
 }  // namespace sdft_hip

@@ -19,8 +19,9 @@ struct GridPlanDev {
   // x-lines that hold sticks, as two ranges [start, start + lines) of natural
   // x: the y-transforms of the local H run on these lines only
   int xstart[2] = {0, 0}, xlines[2] = {0, 0};
-  // no stick has y in [ylow, yhigh)
-  int ylow = 0, yhigh = 0;
+  // no stick has y in [ylow, yhigh), none an entry with z in [zlow, zhigh)
+  int ylow = 0, yhigh = 0, zlow = 0, zhigh = 0;
+  long points = 0;  // plane waves
 };
 
 // y(:,c) = T x(:,c) + FFT_fwd(V . FFT_bwd(x(:,c))) / N for c < columns.

@@ -9,6 +9,7 @@
 namespace sdft_hip {
 
 hipError_t prime_module_local_h();
+hipError_t prime_module_sticks();
 hipError_t prime_module_plane_local_f64();
 hipError_t prime_module_plane_local_f32();
 hipError_t prime_module_gemm();

@@ -29,4 +29,13 @@ template <typename T>
 hipError_t launch_plane_local(const GridPlanDev& p, const PlaneLocalPlan& plan, const void* t1, void* t2, long columns,
                               hipStream_t stream);
 
+// z-transforms of the sticks: x(:, c) gathered from the sphere into
+// t1[column][z slot][stick], and back with y = diag .* x + (transform) / count.
+template <typename T>
+hipError_t launch_sticks_backward(const GridPlanDev& p, const double* x, long ldx, long columns, void* t1,
+                                  hipStream_t stream);
+template <typename T>
+hipError_t launch_sticks_forward(const GridPlanDev& p, const void* t2, long columns, const double* x, long ldx,
+                                 const double* diag, double* y, long ldy, hipStream_t stream);
+
 }  // namespace sdft_hip

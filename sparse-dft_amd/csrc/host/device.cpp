@@ -65,6 +65,7 @@ HostGridPlan build_grid_plan(std::array<int, 3> shape, const std::uint64_t* indi
   p.shape = shape;
   p.split = splits_for(shape);
   p.count = long(shape[0]) * shape[1] * shape[2];
+  p.points = long(n);
   const int n2 = shape[2];
   std::vector<std::pair<int, int>> keys;  // (xy, g)
   keys.reserve(n);
@@ -115,6 +116,7 @@ HostGridPlan build_full_plan(std::array<int, 3> shape) {
   p.shape = shape;
   p.split = splits_for(shape);
   p.count = long(shape[0]) * shape[1] * shape[2];
+  p.points = p.count;
   const int planes = shape[0] * shape[1];
   p.stick_xy.resize(planes);
   p.stick_g.resize(std::size_t(p.count));
@@ -130,17 +132,24 @@ void DeviceGrid::upload(const HostGridPlan& h, hipStream_t s) {
   std::vector<int> map(std::size_t(h.shape[0]) * h.shape[1], -1);
   for (std::size_t i = 0; i < h.stick_xy.size(); ++i) map[std::size_t(h.stick_xy[i])] = int(i);
   stick_map.upload(map.data(), map.size(), s);
-  // the widest run of y around the middle of the axis without a stick
-  const int n1 = h.shape[1];
-  std::vector<char> seen(std::size_t(n1), 0);
-  for (int key : h.stick_xy) seen[std::size_t(key % n1)] = 1;
-  dev.ylow = dev.yhigh = n1 / 2;
-  if (seen[std::size_t(n1 / 2)]) {
-    dev.ylow = dev.yhigh = n1;
-  } else {
-    while (dev.ylow > 0 && !seen[std::size_t(dev.ylow - 1)]) --dev.ylow;
-    while (dev.yhigh < n1 && !seen[std::size_t(dev.yhigh)]) ++dev.yhigh;
-  }
+  // the widest run [low, high) of an axis around its middle that `seen` leaves out
+  auto empty_middle = [](const std::vector<char>& seen, int& low, int& high) {
+    const int n = int(seen.size());
+    low = high = n / 2;
+    if (seen[std::size_t(n / 2)]) {
+      low = high = n;
+      return;
+    }
+    while (low > 0 && !seen[std::size_t(low - 1)]) --low;
+    while (high < n && !seen[std::size_t(high)]) ++high;
+  };
+  std::vector<char> y_seen(std::size_t(h.shape[1]), 0), z_seen(std::size_t(h.shape[2]), 0);
+  for (int key : h.stick_xy) y_seen[std::size_t(key % h.shape[1])] = 1;
+  for (std::size_t e = 0; e < h.stick_g.size(); ++e)
+    if (h.stick_g[e] >= 0) z_seen[e % std::size_t(h.shape[2])] = 1;
+  empty_middle(y_seen, dev.ylow, dev.yhigh);
+  empty_middle(z_seen, dev.zlow, dev.zhigh);
+  dev.points = h.points;
   dev.n0 = h.shape[0];
   dev.n1 = h.shape[1];
   dev.n2 = h.shape[2];
@@ -188,7 +197,7 @@ void prime_libraries(int device) {
   std::lock_guard<std::mutex> lock(m);
   if (std::find(primed.begin(), primed.end(), device) != primed.end()) return;
   rocblas_initialize();
-  for (hipError_t (*f)() : {prime_module_local_h, prime_module_plane_local_f64,
+  for (hipError_t (*f)() : {prime_module_local_h, prime_module_sticks, prime_module_plane_local_f64,
                             prime_module_plane_local_f32, prime_module_gemm, prime_module_davidson_kernels,
                             prime_module_tridiag, prime_module_tridiag_eig, prime_module_realspace,
                             prime_module_batch})

@@ -86,7 +86,7 @@ struct HostGridPlan {
   std::array<int, 3> split{};
   std::vector<int> stick_xy;  // nsticks
   std::vector<int> stick_g;   // nsticks * n2
-  long count = 0;
+  long count = 0, points = 0;    // grid points, plane waves
   int xstart[2]{}, xlines[2]{};  // x-lines holding sticks (two ranges of natural x)
   int nsticks() const { return int(stick_xy.size()); }
 };

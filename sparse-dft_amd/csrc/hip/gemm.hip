@@ -1,7 +1,8 @@
 // Complex GEMM on CDNA4 matrix cores, column-major with explicit leading
 // dimensions (the semantics of src/compute_backend.hpp:21-27):
 //   C = op(A) op(B) + beta * D,  op in {Normal, Adjoint},  D may alias C.
-// Complex products use three real MFMAs per 16x16x4 block (Gauss form, below):
+// Complex products use three real MFMAs per 16x16x4 block (Gauss form, 25 % fewer
+// MFMA cycles than four):
 //   P1 = Ar Br, P2 = Ai Bi, P3 = (Ar + Ai)(Br + Bi); re = P1 - P2, im = P3 - P1 - P2.
 // FP64 uses v_mfma_f64_16x16x4_f64, FP32 uses v_mfma_f32_16x16x4_f32 (inputs
 // stored in FP64 or FP32 are converted while staging into LDS).
@@ -12,11 +13,12 @@
 #include "gemm.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace sdft_hip {
 
 namespace {
-constexpr int BK = 16;  // K slab per LDS round
+constexpr int BK = 16;  // K of one slab
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
@@ -37,19 +39,6 @@ struct Acc<float> {
   }
 };
 
-template <typename S>
-__device__ __forceinline__ void load2(const S* p, double& re, double& im) {
-  re = double(p[0]);
-  im = double(p[1]);
-}
-
-// One BM x BN output tile per 256-thread workgroup (4 waves, WGM along M),
-// K range [k0, k1) of this split. Each wave computes (BM/WGM) x (BN/(4/WGM))
-// as 16 x 16 blocks; per 4-deep K step it first issues the independent
-// Ar*Br / Ar*Bi products of every block, then the dependent -Ai*Bi / Ai*Br
-// ones, so that no MFMA waits on the accumulator of the one just issued.
-// PF: the next K slab is loaded into registers while the current one is
-// multiplied from LDS.
 // XCD-aware tile order. Workgroups are dispatched round-robin over the eight
 // XCDs (linear id L runs on XCD L % 8), each with its own L2. The bijection
 // below hands every XCD a contiguous range of tiles in (split, m, n) order
@@ -69,203 +58,190 @@ __device__ __forceinline__ TileId xcd_tile(int mt, int nt, int splits) {
   return {(t / nt) % mt, t % nt, t / (nt * mt)};
 }
 
-// Complex products as three real MFMA products (Gauss / 3M: Ar Br, Ai Bi,
-// (Ar + Ai)(Br + Bi)) instead of four, 25 % fewer MFMA cycles, in both
-// precisions; SDFT_GEMM_GAUSS_FP64=0 / SDFT_GEMM_GAUSS_FP32=0 build the
-// four-product form.
-#ifndef SDFT_GEMM_GAUSS_FP64
-#define SDFT_GEMM_GAUSS_FP64 1
-#endif
-#ifndef SDFT_GEMM_GAUSS_FP32
-#define SDFT_GEMM_GAUSS_FP32 1
-#endif
+template <typename T>
+struct alignas(2 * sizeof(T)) Pair {
+  T re, im;
+};
 
-// WAVES: at least that many waves per SIMD. Left alone, the FP64 tiles keep
-// their accumulators in AGPRs and the alpha/beta epilogue copies them all to
-// VGPRs at once, which caps occupancy at two waves; the 3M tiles hold a third
-// accumulator set, which fits three waves only in the split-K plan.
-template <typename T, typename TA, typename TB, bool ADJ_A, bool ADJ_B, int TBM, int TBN, int WGM, bool PF, int WAVES>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_zgemm(int M, int N, int K, const TA* __restrict__ A, long lda,
-                                               const TB* __restrict__ B, long ldb, double* __restrict__ C, long ldc,
-                                               const double* __restrict__ D, long ldd, double alpha, double beta,
-                                               int kps, double* __restrict__ work) {
-  constexpr int WGN = 4 / WGM, WM = TBM / WGM, WN = TBN / WGN, IM = WM / 16, JN = WN / 16;
-  constexpr int EA = TBM * BK / 256, EB = TBN * BK / 256;
-  static_assert(EA * 256 == TBM * BK && EB * 256 == TBN * BK, "staging must tile the workgroup");
-  // LDS staging, conflict-free in both directions: an operand whose global
-  // layout runs along K (adjoint A, normal B) is loaded by lanes along K and
-  // kept [m][k] with row stride BK + 1; the other one is loaded along m and
-  // kept [k][m] with row stride TBM + 16 (two K rows of one half-wave read
-  // land on disjoint banks).
-  constexpr int SA = ADJ_A ? BK + 1 : TBM + 16, SB = ADJ_B ? TBN + 16 : BK + 1;
-  constexpr int LA = ADJ_A ? TBM * SA : BK * SA, LB = ADJ_B ? BK * SB : TBN * SB;
-  __shared__ T as_re[LA], as_im[LA];
-  __shared__ T bs_re[LB], bs_im[LB];
-  auto aix = [](int kk, int mm) { return ADJ_A ? mm * SA + kk : kk * SA + mm; };
-  auto bix = [](int kk, int nn) { return ADJ_B ? kk * SB + nn : nn * SB + kk; };
+// One operand's K slab: TM lines (rows of op(A), columns of op(B)) by BK of K, on
+// its way from memory through registers to LDS. ALONG_K: contiguous along K in
+// memory, kept [line][k] with an odd stride; otherwise contiguous along the
+// lines, kept [k][line]. A thread's elements keep their byte offsets for the
+// whole product while the slab's base advances as a scalar. Lines past the edge
+// and k past the end read zeros: past the buffer by the hardware's bounds check.
+// FAR (a leading dimension over kFarStride): 64-bit offsets and a test instead.
+constexpr long kFarStride = 1L << 20;
+template <typename T, typename S, bool ALONG_K, int TM, bool FAR>
+struct Slab {
+  static constexpr int E = TM * BK / 256;
+  static_assert(E * 256 == TM * BK, "staging must tile the workgroup");
+  static constexpr int STRIDE = ALONG_K ? BK + 1 : TM + (sizeof(T) == 8 ? 2 : 16);
+  static constexpr int SIZE = ALONG_K ? TM * STRIDE : BK * STRIDE;
+  using Value = typename std::conditional<sizeof(S) == 8, double2, float2>::type;
+  using Offset = typename std::conditional<FAR, long, int>::type;
+  static constexpr Offset kOut = -16;
+  Value reg[E];
+  Offset off[E];
+  static __device__ __forceinline__ int line_of(int tid, int it) {
+    const int e = tid + it * 256;
+    return ALONG_K ? e / BK : e % TM;
+  }
+  static __device__ __forceinline__ int k_of(int tid, int it) {
+    const int e = tid + it * 256;
+    return ALONG_K ? e % BK : e / TM;
+  }
+  static __device__ __forceinline__ int at(int line, int k) { return ALONG_K ? line * STRIDE + k : k * STRIDE + line; }
+  __device__ __forceinline__ void init(int tid, int lines, long ld) {
+#pragma unroll
+    for (int it = 0; it < E; ++it) {
+      const int l = line_of(tid, it), k = k_of(tid, it);
+      off[it] = l < lines ? Offset((ALONG_K ? l * ld + k : k * ld + l) * long(sizeof(Value))) : kOut;
+    }
+  }
+  static __device__ __forceinline__ Value fetch(const S* base, Offset o) {
+    if constexpr (FAR) {
+      return o >= 0 ? *reinterpret_cast<const Value*>(reinterpret_cast<const char*>(base) + o) : Value{0, 0};
+    } else {
+      const __amdgpu_buffer_rsrc_t r =
+          __builtin_amdgcn_make_buffer_rsrc(const_cast<S*>(base), 0, 0x7fffffff, 0x00027000);
+      if constexpr (sizeof(S) == 8)
+        return __builtin_bit_cast(Value, __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, 0));
+      else
+        return __builtin_bit_cast(Value, __builtin_amdgcn_raw_buffer_load_b64(r, o, 0, 0));
+    }
+  }
+  // `rest`: K left from the slab's start
+  __device__ __forceinline__ void load(const S* base, int tid, int rest) {
+    if (rest >= BK) {
+#pragma unroll
+      for (int it = 0; it < E; ++it) reg[it] = fetch(base, off[it]);
+    } else {
+#pragma unroll
+      for (int it = 0; it < E; ++it) reg[it] = fetch(base, k_of(tid, it) < rest ? off[it] : kOut);
+    }
+  }
+  template <bool CONJ>
+  __device__ __forceinline__ void store(Pair<T>* lds, int tid) {
+#pragma unroll
+    for (int it = 0; it < E; ++it)
+      lds[at(line_of(tid, it), k_of(tid, it))] = Pair<T>{T(reg[it].x), CONJ ? -T(reg[it].y) : T(reg[it].y)};
+  }
+};
+
+// Workgroup barrier over LDS data only: the next slab's loads stay in flight
+// (__syncthreads waits for them). 0xC07F: lgkmcnt(0), the other counters free.
+__device__ __forceinline__ void slab_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// One TBM x TBN output tile per 256-thread workgroup (2 x 2 waves), K range
+// [k0, k1) of this split. Each wave computes (TBM/2) x (TBN/2) as 16 x 16 blocks:
+// per 4-deep K step one LDS read an operand block (re and im together) and three
+// MFMAs a block pair, independent accumulators first. Two LDS slabs: while one is
+// multiplied, the next travels from memory to registers and then into the other,
+// with one barrier a slab. The MFMA takes the operands exchanged (C^T = B^T A^T),
+// so that a lane's results lie along M: stores of 256 contiguous bytes.
+// Bound: FP64 by the MFMA rate at the clock that FP64 MFMA load leaves (near
+// 2.0 GHz: 78 % of the CU's cycles issue MFMAs); FP32 70 % of them. WAVES: at
+// least that many waves per SIMD.
+template <typename T, typename TA, typename TB, bool ADJ_A, bool ADJ_B, int TBM, int TBN, bool FAR, int WAVES>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_zgemm(
+    int M, int N, int K, const TA* __restrict__ A, long lda, const TB* __restrict__ B, long ldb, double* __restrict__ C,
+    long ldc, const double* __restrict__ D, long ldd, double alpha, double beta, int kps, double* __restrict__ work) {
+  constexpr int IM = TBM / 32, JN = TBN / 32;
   using V = typename Acc<T>::type;
+  using SlabA = Slab<T, TA, ADJ_A, TBM, FAR>;
+  using SlabB = Slab<T, TB, !ADJ_B, TBN, FAR>;
+  __shared__ Pair<T> lds_a[2][SlabA::SIZE];
+  __shared__ Pair<T> lds_b[2][SlabB::SIZE];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const TileId tile = xcd_tile(gridDim.x, gridDim.y, gridDim.z);
   const int m0 = tile.m * TBM, n0 = tile.n * TBN;
   const int k0 = tile.split * kps, k1 = min(K, k0 + kps);
-  const int wm = (wave % WGM) * WM, wn = (wave / WGM) * WN;
-  // kGauss: three real products per block (Gauss / 3M),
+  const int wm = (wave & 1) * IM * 16, wn = (wave >> 1) * JN * 16;
   // acc_re = sum Ar Br, acc_x = sum Ai Bi, acc_im = sum (Ar + Ai)(Br + Bi)
-  constexpr bool kGauss = sizeof(T) == 8 ? SDFT_GEMM_GAUSS_FP64 : SDFT_GEMM_GAUSS_FP32;
-  constexpr int GI = kGauss ? IM : 1, GJ = kGauss ? JN : 1;
-  V acc_re[IM][JN], acc_im[IM][JN], acc_x[GI][GJ];
+  V acc_re[IM][JN], acc_im[IM][JN], acc_x[IM][JN];
 #pragma unroll
   for (int i = 0; i < IM; ++i)
 #pragma unroll
-    for (int j = 0; j < JN; ++j) {
-      acc_re[i][j] = V{0, 0, 0, 0};
-      acc_im[i][j] = V{0, 0, 0, 0};
-    }
-#pragma unroll
-  for (int i = 0; i < GI; ++i)
-#pragma unroll
-    for (int j = 0; j < GJ; ++j) acc_x[i][j] = V{0, 0, 0, 0};
-  double pa[EA][2], pb[EB][2];
-  // A_eff[m][k] and B_eff[k][n] of the K slab at kb into registers
-  auto load = [&](int kb) {
-#pragma unroll
-    for (int it = 0; it < EA; ++it) {
-      const int e = tid + it * 256;
-      int mm, kk;
-      if (!ADJ_A) { mm = e % TBM; kk = e / TBM; } else { kk = e % BK; mm = e / BK; }
-      const int m = m0 + mm, k = kb + kk;
-      double re = 0, im = 0;
-      if (m < M && k < k1) {
-        if (!ADJ_A) load2(A + 2 * (m + (long)k * lda), re, im);
-        else { load2(A + 2 * (k + (long)m * lda), re, im); im = -im; }
-      }
-      pa[it][0] = re;
-      pa[it][1] = im;
-    }
-#pragma unroll
-    for (int it = 0; it < EB; ++it) {
-      const int e = tid + it * 256;
-      int nn, kk;
-      if (!ADJ_B) { kk = e % BK; nn = e / BK; } else { nn = e % TBN; kk = e / TBN; }
-      const int n = n0 + nn, k = kb + kk;
-      double re = 0, im = 0;
-      if (n < N && k < k1) {
-        if (!ADJ_B) load2(B + 2 * (k + (long)n * ldb), re, im);
-        else { load2(B + 2 * (n + (long)k * ldb), re, im); im = -im; }
-      }
-      pb[it][0] = re;
-      pb[it][1] = im;
-    }
-  };
-  auto store = [&]() {
-#pragma unroll
-    for (int it = 0; it < EA; ++it) {
-      const int e = tid + it * 256;
-      int mm, kk;
-      if (!ADJ_A) { mm = e % TBM; kk = e / TBM; } else { kk = e % BK; mm = e / BK; }
-      as_re[aix(kk, mm)] = T(pa[it][0]);
-      as_im[aix(kk, mm)] = T(pa[it][1]);
-    }
-#pragma unroll
-    for (int it = 0; it < EB; ++it) {
-      const int e = tid + it * 256;
-      int nn, kk;
-      if (!ADJ_B) { kk = e % BK; nn = e / BK; } else { nn = e % TBN; kk = e / TBN; }
-      bs_re[bix(kk, nn)] = T(pb[it][0]);
-      bs_im[bix(kk, nn)] = T(pb[it][1]);
-    }
-  };
-  if (PF && k0 < k1) load(k0);
+    for (int j = 0; j < JN; ++j) acc_re[i][j] = acc_im[i][j] = acc_x[i][j] = V{0, 0, 0, 0};
+  SlabA sa;
+  SlabB sb;
+  sa.init(tid, M - m0, lda);
+  sb.init(tid, N - n0, ldb);
+  const TA* pa = A + 2 * (ADJ_A ? (long)m0 * lda + k0 : m0 + (long)k0 * lda);
+  const TB* pb = B + 2 * (ADJ_B ? n0 + (long)k0 * ldb : (long)n0 * ldb + k0);
+  const long step_a = 2 * (ADJ_A ? (long)BK : BK * lda), step_b = 2 * (ADJ_B ? BK * ldb : (long)BK);
+  sa.load(pa, tid, k1 - k0);
+  sb.load(pb, tid, k1 - k0);
+  sa.template store<ADJ_A>(lds_a[0], tid);
+  sb.template store<ADJ_B>(lds_b[0], tid);
+  slab_barrier();
+  int buffer = 0;
   for (int kb = k0; kb < k1; kb += BK) {
-    if (!PF) load(kb);
-    store();
-    __syncthreads();
-    if (PF && kb + BK < k1) load(kb + BK);
+    const bool more = kb + BK < k1;
+    if (more) {
+      pa += step_a;
+      pb += step_b;
+      sa.load(pa, tid, k1 - kb - BK);
+      sb.load(pb, tid, k1 - kb - BK);
+    }
+    const Pair<T>* la = lds_a[buffer];
+    const Pair<T>* lb = lds_b[buffer];
 #pragma unroll
     for (int ks = 0; ks < BK; ks += 4) {
       const int kr = ks + (lane >> 4), c = lane & 15;
-      T ar[IM], ai[IM], br[JN], bi[JN];
+      Pair<T> a[IM], b[JN];
 #pragma unroll
-      for (int i = 0; i < IM; ++i) {
-        ar[i] = as_re[aix(kr, wm + 16 * i + c)];
-        ai[i] = as_im[aix(kr, wm + 16 * i + c)];
-      }
+      for (int i = 0; i < IM; ++i) a[i] = la[SlabA::at(wm + 16 * i + c, kr)];
 #pragma unroll
-      for (int j = 0; j < JN; ++j) {
-        br[j] = bs_re[bix(kr, wn + 16 * j + c)];
-        bi[j] = bs_im[bix(kr, wn + 16 * j + c)];
-      }
-      if constexpr (kGauss) {
-        T as[IM], bsum[JN];
+      for (int j = 0; j < JN; ++j) b[j] = lb[SlabB::at(wn + 16 * j + c, kr)];
 #pragma unroll
-        for (int i = 0; i < IM; ++i) as[i] = ar[i] + ai[i];
+      for (int i = 0; i < IM; ++i)
 #pragma unroll
-        for (int j = 0; j < JN; ++j) bsum[j] = br[j] + bi[j];
+        for (int j = 0; j < JN; ++j) {
+          acc_re[i][j] = Acc<T>::mfma(b[j].re, a[i].re, acc_re[i][j]);
+          acc_x[i][j] = Acc<T>::mfma(b[j].im, a[i].im, acc_x[i][j]);
+        }
 #pragma unroll
-        for (int i = 0; i < IM; ++i)
+      for (int i = 0; i < IM; ++i)
 #pragma unroll
-          for (int j = 0; j < JN; ++j) {
-            acc_re[i][j] = Acc<T>::mfma(ar[i], br[j], acc_re[i][j]);
-            acc_im[i][j] = Acc<T>::mfma(as[i], bsum[j], acc_im[i][j]);
-          }
-#pragma unroll
-        for (int i = 0; i < GI; ++i)
-#pragma unroll
-          for (int j = 0; j < GJ; ++j) acc_x[i][j] = Acc<T>::mfma(ai[i], bi[j], acc_x[i][j]);
-      } else {
-#pragma unroll
-        for (int i = 0; i < IM; ++i)
-#pragma unroll
-          for (int j = 0; j < JN; ++j) {
-            acc_re[i][j] = Acc<T>::mfma(ar[i], br[j], acc_re[i][j]);
-            acc_im[i][j] = Acc<T>::mfma(ar[i], bi[j], acc_im[i][j]);
-          }
-#pragma unroll
-        for (int i = 0; i < IM; ++i)
-#pragma unroll
-          for (int j = 0; j < JN; ++j) {
-            acc_re[i][j] = Acc<T>::mfma(-ai[i], bi[j], acc_re[i][j]);
-            acc_im[i][j] = Acc<T>::mfma(ai[i], br[j], acc_im[i][j]);
-          }
-      }
+        for (int j = 0; j < JN; ++j)
+          acc_im[i][j] = Acc<T>::mfma(b[j].re + b[j].im, a[i].re + a[i].im, acc_im[i][j]);
     }
-    __syncthreads();
+    if (more) {
+      buffer ^= 1;
+      sa.template store<ADJ_A>(lds_a[buffer], tid);
+      sb.template store<ADJ_B>(lds_b[buffer], tid);
+      slab_barrier();
+    }
   }
-  // Accumulator layout of each 16x16 block, column lane % 16 in both cases:
-  //   f32 16x16x4: register r holds row 4*(lane/16) + r
-  //   f64 16x16x4: register r holds row 4*r + lane/16
-  const bool split = work != nullptr;
+  // Accumulator layout of each 16x16 block (columns of C^T = rows of C along the
+  // lanes, lane % 16): f32 register r holds column 4*(lane/16) + r of C, f64
+  // column 4*r + lane/16
 #pragma unroll
   for (int i = 0; i < IM; ++i)
 #pragma unroll
     for (int j = 0; j < JN; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = sizeof(T) == 8 ? 4 * r + (lane >> 4) : 4 * (lane >> 4) + r;
-        const int m = m0 + wm + 16 * i + row;
-        const int n = n0 + wn + 16 * j + (lane & 15);
+        const int m = m0 + wm + 16 * i + (lane & 15);
+        const int n = n0 + wn + 16 * j + (sizeof(T) == 8 ? 4 * r + (lane >> 4) : 4 * (lane >> 4) + r);
         if (m >= M || n >= N) continue;
-        double re = double(acc_re[i][j][r]), im = double(acc_im[i][j][r]);
-        if constexpr (kGauss) {
-          const double s2 = double(acc_x[kGauss ? i : 0][kGauss ? j : 0][r]);
-          im = im - re - s2;
-          re = re - s2;
-        }
-        re *= alpha;
-        im *= alpha;
-        if (split) {
-          double* w = work + 2 * ((long)tile.split * M * N + m + (long)n * M);
-          w[0] = re;
-          w[1] = im;
+        const double p1 = double(acc_re[i][j][r]), p2 = double(acc_x[i][j][r]);
+        double re = (p1 - p2) * alpha, im = (double(acc_im[i][j][r]) - p1 - p2) * alpha;
+        if (work) {
+          *reinterpret_cast<double2*>(work + 2 * ((long)tile.split * M * N + m + (long)n * M)) = double2{re, im};
         } else {
           if (beta != 0.0) {
-            const double* d = D + 2 * (m + (long)n * ldd);
-            re += beta * d[0];
-            im += beta * d[1];
+            const double2 d = *reinterpret_cast<const double2*>(D + 2 * (m + (long)n * ldd));
+            re += beta * d.x;
+            im += beta * d.y;
           }
-          double* c = C + 2 * (m + (long)n * ldc);
-          c[0] = re;
-          c[1] = im;
+          *reinterpret_cast<double2*>(C + 2 * (m + (long)n * ldc)) = double2{re, im};
         }
       }
 }
@@ -385,37 +361,21 @@ __global__ void k_atom_blocks_f32(int np, int columns, int atoms, const int* __r
   }
 }
 
-// Tile configurations, both precisions, with register prefetch: 0 = 128 x 32
-// (tall, narrow outputs with normal A: rotations), 1 = 32 x 32 (every other
-// shape: one 16 x 16 block per wave, the most workgroups). Measured on the Si64
-// shapes, 32 x 32 / 64 x 32 / 64 x 64 (or 128 x 32), FP64 with the split counts
-// of fp64_splits: slabs V^H W 800 x 160 x n 57.6 / 46.3 / 39.8 TFLOP/s,
-// back-projections n x 160 x 512 63.4 / 57.9 / 42.2, Gram 160 x 160 x n
-// 42.4 / 39.2 / 30.0, Rayleigh-Ritz 800^3 55.6 / 47.9 / 37.0, projections
-// 512 x 160 x n 65.8 / 66.8 / 55.0, rotations n x 160 x 800 67.7 / - / 67.6;
-// FP32 (four real products, best split count of each): slabs 75.3 / 69.9 /
-// 68.3, back-projections 82.0 / 77.8 / 72.2, Gram 53.2 / 47.4 / 40.1,
-// Rayleigh-Ritz 68.1 / 59.4 / 59.5, projections 82.6 / 88.1 / 79.7, rotations
-// 86.0 / 89.2 / 77.8 (128 x 32: 90.5).
+// Tiles: 0 = 32 x 32, 1 = 64 x 32, 2 = 64 x 64.
 struct Tile {
   int bm, bn;
 };
-constexpr Tile kTiles[2] = {{128, 32}, {32, 32}};
+constexpr Tile kTiles[3] = {{32, 32}, {64, 32}, {64, 64}};
 
-bool tall_shape(int M, int N) { return M >= 2048 && N <= 192 && long(M) >= 8L * N; }
-
-template <typename T, typename TA, typename TB, int CFG>
+template <typename T, typename TA, typename TB, int CFG, bool FAR>
 hipError_t launch_cfg(int aop, int bop, dim3 grid, int M, int N, int K, const TA* A, long lda, const TB* B, long ldb,
                       double* C, long ldc, const double* D, long ldd, double alpha, double beta, int kps,
                       double* work, hipStream_t s) {
-  constexpr int TBM = kTiles[CFG].bm, TBN = kTiles[CFG].bn, WGM = CFG == 0 ? 4 : 2;
-  constexpr bool PF = true;
-  // measured on the Si64 shapes: the 3M FP64 tiles at two waves per SIMD
-  // (three spill), the FP32 tiles at three
-  constexpr int WAVES = (sizeof(T) == 8 && SDFT_GEMM_GAUSS_FP64) ? 2 : 3;
-#define SDFT_LAUNCH(AA, BB)                                                                                      \
-  hipLaunchKernelGGL((k_zgemm<T, TA, TB, AA, BB, TBM, TBN, WGM, PF, WAVES>), grid, dim3(256), 0, s, M, N, K, A, \
-                     lda, B, ldb, C, ldc, D, ldd, alpha, beta, kps, work)
+  constexpr int TBM = kTiles[CFG].bm, TBN = kTiles[CFG].bn;
+  constexpr int WAVES = sizeof(T) == 4 && CFG == 0 ? 3 : 2;
+#define SDFT_LAUNCH(AA, BB)                                                                                         \
+  hipLaunchKernelGGL((k_zgemm<T, TA, TB, AA, BB, TBM, TBN, FAR, WAVES>), grid, dim3(256), 0, s, M, N, K, A, lda, B, \
+                     ldb, C, ldc, D, ldd, alpha, beta, kps, work)
   if (!aop && !bop) SDFT_LAUNCH(false, false);
   else if (aop && !bop) SDFT_LAUNCH(true, false);
   else if (!aop && bop) SDFT_LAUNCH(false, true);
@@ -433,8 +393,17 @@ hipError_t dispatch_ops(int cfg, int aop, int bop, dim3 grid, int M, int N, int 
     if (e != hipSuccess) return e;
   }
   hipError_t e;
-  if (cfg == 0) e = launch_cfg<T, TA, TB, 0>(aop, bop, grid, M, N, K, A, lda, B, ldb, C, ldc, D, ldd, alpha, beta, kps, work, s);
-  else e = launch_cfg<T, TA, TB, 1>(aop, bop, grid, M, N, K, A, lda, B, ldb, C, ldc, D, ldd, alpha, beta, kps, work, s);
+  if (lda > kFarStride || ldb > kFarStride) {
+    // 32-bit byte offsets do not reach a tile's last line: 64-bit ones, 32 x 32
+    const dim3 far((M + 31) / 32, (N + 31) / 32, grid.z);
+    e = launch_cfg<T, TA, TB, 0, true>(aop, bop, far, M, N, K, A, lda, B, ldb, C, ldc, D, ldd, alpha, beta, kps, work, s);
+  } else if (cfg == 2) {
+    e = launch_cfg<T, TA, TB, 2, false>(aop, bop, grid, M, N, K, A, lda, B, ldb, C, ldc, D, ldd, alpha, beta, kps, work, s);
+  } else if (cfg == 1) {
+    e = launch_cfg<T, TA, TB, 1, false>(aop, bop, grid, M, N, K, A, lda, B, ldb, C, ldc, D, ldd, alpha, beta, kps, work, s);
+  } else {
+    e = launch_cfg<T, TA, TB, 0, false>(aop, bop, grid, M, N, K, A, lda, B, ldb, C, ldc, D, ldd, alpha, beta, kps, work, s);
+  }
   if (e != hipSuccess || !ev || !ev->end) return e;
   return hipEventRecord(ev->end, s);
 }
@@ -444,54 +413,61 @@ struct Plan {
   int cfg, splits, kps;
   dim3 grid;
 };
-// splits along K: double while the workgroups number fewer than `target` and
-// every split keeps >= 256 of K
-int splits_for(long tiles, int K, long target) {
-  int splits = 1;
-  while (tiles * splits < target && long(K) / (2 * splits) >= 256 && splits < 64) splits *= 2;
-  return splits;
-}
 long tile_count(int M, int N, int cfg) {
   return long((M + kTiles[cfg].bm - 1) / kTiles[cfg].bm) * ((N + kTiles[cfg].bn - 1) / kTiles[cfg].bn);
 }
-// 32 x 32 tiles split along K to >= 2048 (FP64) or >= 1024 (FP32)
-// workgroups, tall shapes to >= 512 (they need no split); rotations (tall,
-// normal A) 128 x 32
-int plan_cfg(int M, int N, int aop) { return tall_shape(M, N) && !aop ? 0 : 1; }
-int plan_splits(bool fp64, int M, int N, int K, int aop) {
-  const int cfg = plan_cfg(M, N, aop);
-  return splits_for(tile_count(M, N, cfg), K, tall_shape(M, N) ? 512 : fp64 ? 2048 : 1024);
+// Splits along K for about 1200 workgroups (a little over four a CU; 512 x 160 x n took
+// 213 us with 1280, 230 and more with 640), at least 256 of K each, or 128 while that
+// leaves CUs without a workgroup (128 x 37 x 4573 in 32 splits of 143); 48 at most.
+int splits_for(long tiles, int K) {
+  const long most = std::min<long>(48, (1200 + tiles - 1) / tiles);
+  long splits = std::min<long>(most, std::max<long>(1, K / 256));
+  if (tiles * splits < 256) splits = std::min<long>(most, std::max<long>(1, K / 128));
+  return int(std::max<long>(1, splits));
 }
-Plan plan_for(bool fp64, int aop, int M, int N, int K, bool have_work) {
+// The tile of a shape, for both precisions: 64 x 64 where the result is wide (256
+// columns, at most a tenth of them padding) and has 1200 such tiles, 64 x 32 where
+// 768 workgroups are reached with splits, else 32 x 32. Measured, us, 64 x 64 /
+// 64 x 32 / 32 x 32 at their best splits (n = 23847): n x 480 x 512 adjoint FP64
+// 687 / 749 / 777, FP32 373 / 433 / 494; 512 x 160 x n FP64 268 / 213 / 225, FP32
+// 140 / 126 / 133; 640 x 160 x n FP64 331 / 299 / 299, FP32 183 / 176 / 197; n x 220 x
+// 380 FP64 279 / 260 / 267; 160 x 160 x n FP64 116 / 95 / 85; 128 x 37 x 4573 FP64
+// 25 / 17 / 13; 9141 x 80 x 256 adjoint FP64 57 / 38 / 37. Against the single-buffered
+// kernels (32 x 32 and 128 x 32 tiles, two barriers and per-element addresses and
+// bounds in every slab): 512 x 160 x n FP64 287, FP32 164; 640 x 160 x n 391, 236;
+// n x 480 x 512 823, 562; 160 x 160 x n 101, 69; 128 x 37 x 4573 19, 16.
+Plan plan_shape(int M, int N, int K) {
   Plan p{};
-  p.splits = plan_splits(fp64, M, N, K, aop);
+  p.cfg = 0;
+  if (N >= 256 && (N + 63) / 64 * 64 <= N + N / 10 && tile_count(M, N, 2) >= 1200) {
+    p.cfg = 2;
+  } else {
+    const long tiles = tile_count(M, N, 1);
+    if (tiles * splits_for(tiles, K) >= 768) p.cfg = 1;
+  }
+  p.splits = splits_for(tile_count(M, N, p.cfg), K);
+  return p;
+}
+Plan plan_for(int M, int N, int K, bool have_work) {
+  Plan p = plan_shape(M, N, K);
   if (p.splits > 1 && !have_work) p.splits = 1;
   p.kps = (K + p.splits - 1) / p.splits;
   p.kps = ((p.kps + BK - 1) / BK) * BK;
   p.splits = (K + p.kps - 1) / p.kps;
-  p.cfg = plan_cfg(M, N, aop);
   p.grid = dim3((M + kTiles[p.cfg].bm - 1) / kTiles[p.cfg].bm, (N + kTiles[p.cfg].bn - 1) / kTiles[p.cfg].bn,
                 p.splits);
   return p;
 }
 }  // namespace
 
-int zgemm_real_products(Precision prec) {
-  return (prec == Precision::FP64 ? SDFT_GEMM_GAUSS_FP64 : SDFT_GEMM_GAUSS_FP32) ? 3 : 4;
-}
+int zgemm_real_products(Precision) { return 3; }
 
 std::size_t zgemm_workspace_bytes(int M, int N, int K) {
   const int splits = zgemm_splits(M, N, K);
   return splits > 1 ? std::size_t(splits) * M * N * 16 : 0;
 }
 
-// the largest split count any plan of the shape uses (workspace sizing)
-int zgemm_splits(int M, int N, int K) {
-  int splits = 1;
-  for (int aop = 0; aop < 2; ++aop)
-    for (int fp64 = 0; fp64 < 2; ++fp64) splits = std::max(splits, plan_splits(fp64, M, N, K, aop));
-  return splits;
-}
+int zgemm_splits(int M, int N, int K) { return K > 0 ? plan_shape(M, N, K).splits : 1; }
 
 hipError_t zgemm(Precision prec, int aop, int bop, int M, int N, int K, double alpha, const double* A, long lda,
                  const double* B, long ldb, double* C, long ldc, const double* D, long ldd, double beta, double* work,
@@ -502,7 +478,7 @@ hipError_t zgemm(Precision prec, int aop, int bop, int M, int N, int K, double a
     return launch_zaxpby(M, N, 0.0, nullptr, 0, beta, D, ldd, C, ldc, s);
   }
   const bool room = work != nullptr && work_bytes >= zgemm_workspace_bytes(M, N, K);
-  const Plan pl = plan_for(prec == Precision::FP64, aop, M, N, K, room);
+  const Plan pl = plan_for(M, N, K, room);
   double* wk = pl.splits > 1 ? work : nullptr;
   hipError_t e;
   if (prec == Precision::FP64)
@@ -521,7 +497,7 @@ hipError_t zgemm_f32_storage(int aop, int bop, int M, int N, int K, double alpha
                              double* work, std::size_t work_bytes, hipStream_t s, const LaunchEvents* ev) {
   if (M <= 0 || N <= 0 || K <= 0) return hipSuccess;
   const bool room = work != nullptr && work_bytes >= zgemm_workspace_bytes(M, N, K);
-  const Plan pl = plan_for(false, aop, M, N, K, room);
+  const Plan pl = plan_for(M, N, K, room);
   double* wk = pl.splits > 1 ? work : nullptr;
   hipError_t e = dispatch_ops<float, float, double>(pl.cfg, aop, bop, pl.grid, M, N, K, A, lda, B, ldb, C, ldc, D, ldd,
                                                     alpha, beta, pl.kps, wk, s, ev);

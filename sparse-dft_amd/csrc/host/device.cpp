@@ -597,6 +597,17 @@ void DeviceOperator::set_chunk() {
   chunk_ = std::max<std::size_t>(1, std::min<std::size_t>(cap, (std::size_t(512) << 20) / std::max<std::size_t>(1, per_col)));
 }
 
+// Columns of one pass over `columns`: passes of equal width (a narrow last pass
+// leaves the GEMMs and the chip half empty: S of 480 columns of 64 atoms took 462
+// and 18), and for S, which has no stick buffers, as many as keep its projections
+// below 512 MiB.
+long DeviceOperator::pass_columns(int which, long columns) const {
+  long most = long(chunk_);
+  if (which == 1) most = std::max(most, std::min(4096L, (512L << 20) / std::max<long>(1, 48 * long(np_))));
+  const long passes = (columns + most - 1) / most;
+  return (columns + passes - 1) / passes;
+}
+
 DeviceOperator::DeviceOperator(Context& ctx, const SnapshotArrays& sa) : ctx_(ctx) {
   n_ = std::size_t(sa.n);
   np_ = std::size_t(sa.projectors);
@@ -751,8 +762,9 @@ void DeviceOperator::apply(int which, const double* x, long columns, double* hy,
     if (which != 0) apply_real_space(1, x, columns, sy, prec);
     return;
   }
-  for (long c0 = 0; c0 < columns; c0 += long(chunk_)) {
-    const long c = std::min<long>(long(chunk_), columns - c0);
+  const long pass = pass_columns(which, columns);
+  for (long c0 = 0; c0 < columns; c0 += pass) {
+    const long c = std::min<long>(pass, columns - c0);
     const long off = 2 * c0 * long(n_);
     apply_chunk(which, x + off, c, hy ? hy + off : nullptr, sy ? sy + off : nullptr, prec,
                 owned_staging(which, c, prec));
@@ -784,8 +796,9 @@ void DeviceOperator::apply_shifted(const double* x, long columns, const double* 
     check(launch_column_scaled_add(sx, long(n_), y, long(n_), long(n_), columns, theta, -1.0, ctx_.stream()),
           "shift");
   } else {
-    for (long c0 = 0; c0 < columns; c0 += long(chunk_)) {
-      const long c = std::min<long>(long(chunk_), columns - c0);
+    const long pass = pass_columns(2, columns);
+    for (long c0 = 0; c0 < columns; c0 += pass) {
+      const long c = std::min<long>(pass, columns - c0);
       const long off = 2 * c0 * long(n_);
       apply_chunk(2, x + off, c, y + off, nullptr, prec, owned_staging(2, c, prec), theta + c0,
                   bf16_projectors && prec != Precision::FP64);
@@ -860,7 +873,7 @@ void DeviceOperator::apply_noalloc(int which, const double* x, long columns, dou
                             "-byte scratch array of the allocation-free apply");
   for (long c0 = 0; c0 < columns;) {
     // the most columns (up to apply()'s chunk) whose staging fits
-    long c = std::min<long>(long(chunk_), columns - c0);
+    long c = std::min<long>(pass_columns(which, columns), columns - c0);
     while (c > 1 && noalloc_bytes(which, c, prec) > kScratchBytes) {
       const double ratio = double(kScratchBytes) / double(noalloc_bytes(which, c, prec));
       c = std::max<long>(1, std::min<long>(c - 1, long(double(c) * ratio)));

@@ -311,6 +311,8 @@ class DeviceOperator {
   // Davidson buffers kept for the next solve are counted by the solver)
   std::size_t device_bytes() const;
   std::size_t max_chunk() const { return chunk_; }
+  // columns of one pass of an application of `columns` columns
+  long pass_columns(int which, long columns) const;
   const GridPlanDev& grid_plan() const { return grid_.dev; }
   // device arrays of the nonlocal part (atom-block form 3): projectors
   // np x n column-major (FP64 and FP32 copies), Hermitised per-atom D and Q

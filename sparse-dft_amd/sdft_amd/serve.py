@@ -132,9 +132,10 @@ def grid_shape(prob):
 def estimate_request_bytes(prob, roots, subspace_factor=8):
     """Upper bound of the device bytes one solve request holds: the operator's
     arrays (V(r) FP64 + FP32, kinetic, projectors FP64 + FP32, onsite blocks,
-    stick plan), its stick and projection work buffers for the largest block
-    a solve applies at once (the subspace capacity, at most the operator's
-    apply chunk), and the Davidson buffers (six n x capacity blocks, seven
+    stick plan), its stick work buffers for the largest block a solve applies
+    at once (the subspace capacity, at most the operator's apply chunk) and
+    its projection buffers for the largest S application (the seed block or
+    the capacity), and the Davidson buffers (six n x capacity blocks, seven
     n x roots blocks, the projected matrices and the Rayleigh-Ritz
     eigensolver), with capacity = min(n, max(factor roots, 64)) as the solver
     sizes it, plus 1 MiB for the small control buffers."""
@@ -149,7 +150,8 @@ def estimate_request_bytes(prob, roots, subspace_factor=8):
     chunk = max(1, min(512, (512 * MiB) // max(per_col, 1)))
     cols = min(max(cap, 2 * roots), chunk)
     operator = (count * 12 + n * 8 + np_ * n * 24 + 2 * 16 * sum(r * r for r in prob.atom_rows) +
-                sticks * (shape[2] + 1) * 4 + 2 * cols * per_col + 3 * 16 * np_ * cols)
+                sticks * (shape[2] + 1) * 4 + shape[0] * shape[1] * 4 + 2 * cols * per_col +
+                3 * 16 * np_ * max(cap, 3 * roots))
     davidson = 16 * (6 * n * cap + 7 * n * roots + 12 * cap * cap + 4 * roots * roots + 8 * (2 * roots) ** 2)
     return operator + davidson + MiB
 

@@ -157,7 +157,10 @@ void OperatorBatch::autotune() {
     std::lock_guard<std::mutex> lock(g_plan_mutex);
     auto it = g_plans.find(key_);
     if (it != g_plans.end()) {
-      launch_ = it->second.first;
+      // only the launch shape: the twiddles belong to this batch's operators
+      launch_.threads = it->second.first.threads;
+      launch_.planes = it->second.first.planes;
+      launch_.groups = it->second.first.groups;
       tuned_ms_ = it->second.second;
       cached_ = true;
       return;

@@ -306,8 +306,8 @@ def main():
     names = {"gemm_fp64": "sdft_hip::k_zgemm<double, ...> (FP64 MFMA complex GEMM, all shapes of the solve)",
              "gemm_fp32": "sdft_hip::k_zgemm<float, ...> (FP32 MFMA complex GEMM, all shapes of the solve)",
              "gemm_bf16": "sdft_hip::k_zgemm_bf16 (BF16 MFMA projector GEMMs of the correction solves)",
-             "local_fp64": "local-H pipeline FP64 (k_sticks_backward + k_planes + k_sticks_forward)",
-             "local_fp32": "local-H pipeline FP32 (k_sticks_backward + k_planes + k_sticks_forward)"}
+             "local_fp64": "local-H pipeline FP64 (k_sticks_backward + k_plane_local + k_sticks_forward)",
+             "local_fp32": "local-H pipeline FP32 (k_sticks_backward + k_plane_local + k_sticks_forward)"}
     kernels = {}
     for k, st in clock.items():
         if not st["launches"]:
@@ -329,11 +329,6 @@ def main():
         if k in products:
             kernels[k]["real_products_per_complex_mac"] = products[k]
             kernels[k]["mfma_executed_frac"] = kernels[k]["frac"] * products[k] / 4
-        else:
-            # inside the solve the local-H pipeline runs on a second stream beside
-            # the projector GEMMs, so its event time includes the CUs it shares;
-            # isolated_local_h times it alone
-            kernels[k]["concurrent_with"] = "projector GEMM chain on the main stream"
     roofline = {"bound": bound, "achieved": kernels[dom]["achieved"], "peak": peak, "unit": unit,
                 "frac": kernels[dom]["frac"], "traffic": traffic, "kernel": names[dom],
                 "work_per_launch": kernels[dom]["work_per_launch"],

@@ -65,7 +65,8 @@ int sdft_hip_synchronize(sdft_hip_context* ctx);
  * GEMM kernel and every local-Hamiltonian pipeline launch. Enabling or
  * disabling clears the sums. kind: 0 GEMM FP64, 1 GEMM FP32 arithmetic,
  * 2 local H FP64, 3 local H FP32, 4 GEMM BF16 arithmetic. work: flops (8 m n k per GEMM) or the
- * algorithmic bytes m (2 npw c + 4 N c) + N r + npw (4 + r) per local-H launch.
+ * algorithmic bytes m (2 npw c + 4 N c) + N r + npw (4 + r) per local-H launch;
+ * launches: products (one GEMM launch that forms H and S images counts as two).
  * The stats call synchronises the stream. */
 #define SDFT_HIP_CLOCK_GEMM_FP64 0
 #define SDFT_HIP_CLOCK_GEMM_FP32 1

@@ -14,6 +14,7 @@
 
 #include <algorithm>
 #include <type_traits>
+#include <vector>
 
 namespace sdft_hip {
 
@@ -149,8 +150,8 @@ __device__ __forceinline__ void slab_barrier() {
 // least that many waves per SIMD.
 template <typename T, typename TA, typename TB, bool ADJ_A, bool ADJ_B, int TBM, int TBN, bool FAR, int WAVES>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_zgemm(
-    int M, int N, int K, const TA* __restrict__ A, long lda, const TB* __restrict__ B, long ldb, double* __restrict__ C,
-    long ldc, const double* __restrict__ D, long ldd, double alpha, double beta, int kps, double* __restrict__ work) {
+    int M, int N, int K, const TA* __restrict__ A, long lda, const TB* __restrict__ B, long ldb, GemmOutput first,
+    GemmOutput second, int n_first, double alpha, int kps, double* __restrict__ work) {
   constexpr int IM = TBM / 32, JN = TBN / 32;
   using V = typename Acc<T>::type;
   using SlabA = Slab<T, TA, ADJ_A, TBM, FAR>;
@@ -236,18 +237,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
         if (work) {
           *reinterpret_cast<double2*>(work + 2 * ((long)tile.split * M * N + m + (long)n * M)) = double2{re, im};
         } else {
-          if (beta != 0.0) {
-            const double2 d = *reinterpret_cast<const double2*>(D + 2 * (m + (long)n * ldd));
-            re += beta * d.x;
-            im += beta * d.y;
+          const bool one = n < n_first;
+          const GemmOutput& o = one ? first : second;
+          const long column = one ? n : n - n_first;
+          if (o.beta != 0.0) {
+            const double2 d = *reinterpret_cast<const double2*>(o.D + 2 * (m + column * o.ldd));
+            re += o.beta * d.x;
+            im += o.beta * d.y;
           }
-          *reinterpret_cast<double2*>(C + 2 * (m + (long)n * ldc)) = double2{re, im};
+          *reinterpret_cast<double2*>(o.C + 2 * (m + column * o.ldc)) = double2{re, im};
         }
       }
 }
 
-__global__ void k_splitk_reduce(int M, int N, int splits, const double* __restrict__ work, double* __restrict__ C,
-                                long ldc, const double* __restrict__ D, long ldd, double beta) {
+__global__ void k_splitk_reduce(int M, int N, int splits, const double* __restrict__ work, GemmOutput first,
+                                GemmOutput second, int n_first) {
   // partials already carry alpha
   const long total = (long)M * N;
   for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < total; e += (long)gridDim.x * blockDim.x) {
@@ -272,12 +276,15 @@ __global__ void k_splitk_reduce(int M, int N, int splits, const double* __restri
       re += w[0];
       im += w[1];
     }
-    if (beta != 0.0) {
-      const double* d = D + 2 * (m + n * ldd);
-      re += beta * d[0];
-      im += beta * d[1];
+    const bool one = n < n_first;
+    const GemmOutput& o = one ? first : second;
+    const long column = one ? n : n - n_first;
+    if (o.beta != 0.0) {
+      const double* d = o.D + 2 * (m + column * o.ldd);
+      re += o.beta * d[0];
+      im += o.beta * d[1];
     }
-    double* c = C + 2 * (m + n * ldc);
+    double* c = o.C + 2 * (m + column * o.ldc);
     c[0] = re;
     c[1] = im;
   }
@@ -369,13 +376,13 @@ constexpr Tile kTiles[3] = {{32, 32}, {64, 32}, {64, 64}};
 
 template <typename T, typename TA, typename TB, int CFG, bool FAR>
 hipError_t launch_cfg(int aop, int bop, dim3 grid, int M, int N, int K, const TA* A, long lda, const TB* B, long ldb,
-                      double* C, long ldc, const double* D, long ldd, double alpha, double beta, int kps,
+                      const GemmOutput& first, const GemmOutput& second, int n_first, double alpha, int kps,
                       double* work, hipStream_t s) {
   constexpr int TBM = kTiles[CFG].bm, TBN = kTiles[CFG].bn;
   constexpr int WAVES = sizeof(T) == 4 && CFG == 0 ? 3 : 2;
 #define SDFT_LAUNCH(AA, BB)                                                                                         \
   hipLaunchKernelGGL((k_zgemm<T, TA, TB, AA, BB, TBM, TBN, FAR, WAVES>), grid, dim3(256), 0, s, M, N, K, A, lda, B, \
-                     ldb, C, ldc, D, ldd, alpha, beta, kps, work)
+                     ldb, first, second, n_first, alpha, kps, work)
   if (!aop && !bop) SDFT_LAUNCH(false, false);
   else if (aop && !bop) SDFT_LAUNCH(true, false);
   else if (!aop && bop) SDFT_LAUNCH(false, true);
@@ -386,7 +393,7 @@ hipError_t launch_cfg(int aop, int bop, dim3 grid, int M, int N, int K, const TA
 
 template <typename T, typename TA, typename TB>
 hipError_t dispatch_ops(int cfg, int aop, int bop, dim3 grid, int M, int N, int K, const TA* A, long lda, const TB* B,
-                        long ldb, double* C, long ldc, const double* D, long ldd, double alpha, double beta, int kps,
+                        long ldb, const GemmOutput& first, const GemmOutput& second, int n_first, double alpha, int kps,
                         double* work, hipStream_t s, const LaunchEvents* ev) {
   if (ev && ev->begin) {
     const hipError_t e = hipEventRecord(ev->begin, s);
@@ -396,13 +403,13 @@ hipError_t dispatch_ops(int cfg, int aop, int bop, dim3 grid, int M, int N, int 
   if (lda > kFarStride || ldb > kFarStride) {
     // 32-bit byte offsets do not reach a tile's last line: 64-bit ones, 32 x 32
     const dim3 far((M + 31) / 32, (N + 31) / 32, grid.z);
-    e = launch_cfg<T, TA, TB, 0, true>(aop, bop, far, M, N, K, A, lda, B, ldb, C, ldc, D, ldd, alpha, beta, kps, work, s);
+    e = launch_cfg<T, TA, TB, 0, true>(aop, bop, far, M, N, K, A, lda, B, ldb, first, second, n_first, alpha, kps, work, s);
   } else if (cfg == 2) {
-    e = launch_cfg<T, TA, TB, 2, false>(aop, bop, grid, M, N, K, A, lda, B, ldb, C, ldc, D, ldd, alpha, beta, kps, work, s);
+    e = launch_cfg<T, TA, TB, 2, false>(aop, bop, grid, M, N, K, A, lda, B, ldb, first, second, n_first, alpha, kps, work, s);
   } else if (cfg == 1) {
-    e = launch_cfg<T, TA, TB, 1, false>(aop, bop, grid, M, N, K, A, lda, B, ldb, C, ldc, D, ldd, alpha, beta, kps, work, s);
+    e = launch_cfg<T, TA, TB, 1, false>(aop, bop, grid, M, N, K, A, lda, B, ldb, first, second, n_first, alpha, kps, work, s);
   } else {
-    e = launch_cfg<T, TA, TB, 0, false>(aop, bop, grid, M, N, K, A, lda, B, ldb, C, ldc, D, ldd, alpha, beta, kps, work, s);
+    e = launch_cfg<T, TA, TB, 0, false>(aop, bop, grid, M, N, K, A, lda, B, ldb, first, second, n_first, alpha, kps, work, s);
   }
   if (e != hipSuccess || !ev || !ev->end) return e;
   return hipEventRecord(ev->end, s);
@@ -469,41 +476,60 @@ std::size_t zgemm_workspace_bytes(int M, int N, int K) {
 
 int zgemm_splits(int M, int N, int K) { return K > 0 ? plan_shape(M, N, K).splits : 1; }
 
-hipError_t zgemm(Precision prec, int aop, int bop, int M, int N, int K, double alpha, const double* A, long lda,
-                 const double* B, long ldb, double* C, long ldc, const double* D, long ldd, double beta, double* work,
-                 std::size_t work_bytes, hipStream_t s, const LaunchEvents* ev) {
-  if (M <= 0 || N <= 0) return hipSuccess;
-  if (K <= 0) {
-    // C = beta * D
-    return launch_zaxpby(M, N, 0.0, nullptr, 0, beta, D, ldd, C, ldc, s);
-  }
+namespace {
+template <typename T, typename TA>
+hipError_t run(int aop, int bop, int M, int N, int K, double alpha, const TA* A, long lda, const double* B, long ldb,
+               const GemmOutput& first, const GemmOutput& second, int n_first, double* work, std::size_t work_bytes,
+               hipStream_t s, const LaunchEvents* ev, int* partials) {
   const bool room = work != nullptr && work_bytes >= zgemm_workspace_bytes(M, N, K);
   const Plan pl = plan_for(M, N, K, room);
   double* wk = pl.splits > 1 ? work : nullptr;
-  hipError_t e;
-  if (prec == Precision::FP64)
-    e = dispatch_ops<double, double, double>(pl.cfg, aop, bop, pl.grid, M, N, K, A, lda, B, ldb, C, ldc, D, ldd, alpha,
-                                             beta, pl.kps, wk, s, ev);
-  else
-    e = dispatch_ops<float, double, double>(pl.cfg, aop, bop, pl.grid, M, N, K, A, lda, B, ldb, C, ldc, D, ldd, alpha,
-                                            beta, pl.kps, wk, s, ev);
-  if (e != hipSuccess || pl.splits == 1) return e;
-  hipLaunchKernelGGL(k_splitk_reduce, dim3(1024), dim3(256), 0, s, M, N, pl.splits, work, C, ldc, D, ldd, beta);
+  const hipError_t e = dispatch_ops<T, TA, double>(pl.cfg, aop, bop, pl.grid, M, N, K, A, lda, B, ldb, first, second,
+                                                   n_first, alpha, pl.kps, wk, s, ev);
+  if (partials) *partials = pl.splits;
+  if (e != hipSuccess || pl.splits == 1 || partials) return e;
+  hipLaunchKernelGGL(k_splitk_reduce, dim3(1024), dim3(256), 0, s, M, N, pl.splits, work, first, second, n_first);
   return hipGetLastError();
+}
+}  // namespace
+
+hipError_t zgemm(Precision prec, int aop, int bop, int M, int N, int K, double alpha, const double* A, long lda,
+                 const double* B, long ldb, double* C, long ldc, const double* D, long ldd, double beta, double* work,
+                 std::size_t work_bytes, hipStream_t s, const LaunchEvents* ev, int* partials) {
+  if (M <= 0 || N <= 0) return hipSuccess;
+  if (K <= 0) {
+    // C = beta * D
+    if (partials) *partials = 1;
+    return launch_zaxpby(M, N, 0.0, nullptr, 0, beta, D, ldd, C, ldc, s);
+  }
+  const GemmOutput o{C, ldc, D, ldd, beta};
+  return prec == Precision::FP64
+             ? run<double, double>(aop, bop, M, N, K, alpha, A, lda, B, ldb, o, o, N, work, work_bytes, s, ev, partials)
+             : run<float, double>(aop, bop, M, N, K, alpha, A, lda, B, ldb, o, o, N, work, work_bytes, s, ev, partials);
 }
 
 hipError_t zgemm_f32_storage(int aop, int bop, int M, int N, int K, double alpha, const float* A, long lda,
                              const double* B, long ldb, double* C, long ldc, const double* D, long ldd, double beta,
-                             double* work, std::size_t work_bytes, hipStream_t s, const LaunchEvents* ev) {
+                             double* work, std::size_t work_bytes, hipStream_t s, const LaunchEvents* ev,
+                             int* partials) {
   if (M <= 0 || N <= 0 || K <= 0) return hipSuccess;
-  const bool room = work != nullptr && work_bytes >= zgemm_workspace_bytes(M, N, K);
-  const Plan pl = plan_for(M, N, K, room);
-  double* wk = pl.splits > 1 ? work : nullptr;
-  hipError_t e = dispatch_ops<float, float, double>(pl.cfg, aop, bop, pl.grid, M, N, K, A, lda, B, ldb, C, ldc, D, ldd,
-                                                    alpha, beta, pl.kps, wk, s, ev);
-  if (e != hipSuccess || pl.splits == 1) return e;
-  hipLaunchKernelGGL(k_splitk_reduce, dim3(1024), dim3(256), 0, s, M, N, pl.splits, work, C, ldc, D, ldd, beta);
-  return hipGetLastError();
+  const GemmOutput o{C, ldc, D, ldd, beta};
+  return run<float, float>(aop, bop, M, N, K, alpha, A, lda, B, ldb, o, o, N, work, work_bytes, s, ev, partials);
+}
+
+hipError_t zgemm_two_outputs(int aop, int M, int n_first, int n_second, int K, const double* A, long lda,
+                             const double* B, long ldb, const GemmOutput& first, const GemmOutput& second, double* work,
+                             std::size_t work_bytes, hipStream_t s, const LaunchEvents* ev) {
+  if (M <= 0 || n_first <= 0 || n_second <= 0 || K <= 0) return hipErrorInvalidValue;
+  return run<double, double>(aop, 0, M, n_first + n_second, K, 1.0, A, lda, B, ldb, first, second, n_first, work,
+                             work_bytes, s, ev, nullptr);
+}
+hipError_t zgemm_two_outputs(int aop, int M, int n_first, int n_second, int K, const float* A, long lda,
+                             const double* B, long ldb, const GemmOutput& first, const GemmOutput& second, double* work,
+                             std::size_t work_bytes, hipStream_t s, const LaunchEvents* ev) {
+  if (M <= 0 || n_first <= 0 || n_second <= 0 || K <= 0) return hipErrorInvalidValue;
+  return run<float, float>(aop, 0, M, n_first + n_second, K, 1.0, A, lda, B, ldb, first, second, n_first, work,
+                           work_bytes, s, ev, nullptr);
 }
 
 // ---- BF16 projector products (search arithmetic) ----
@@ -670,7 +696,8 @@ __global__ void k_to_bf16_pairs(const S* __restrict__ x, long count, unsigned* _
 
 hipError_t zgemm_bf16_storage(int aop, int M, int N, int K, double alpha, const unsigned* A, long lda,
                               const double* B, long ldb, double* C, long ldc, const double* D, long ldd, double beta,
-                              double* work, std::size_t work_bytes, hipStream_t s, const LaunchEvents* ev) {
+                              double* work, std::size_t work_bytes, hipStream_t s, const LaunchEvents* ev,
+                              int* partials) {
   if (M <= 0 || N <= 0 || K <= 0) return hipSuccess;
   const long tiles = long((M + HTBM - 1) / HTBM) * ((N + HTBN - 1) / HTBN);
   // long contractions split along K to >= 512 workgroups, within the workspace
@@ -694,8 +721,10 @@ hipError_t zgemm_bf16_storage(int aop, int M, int N, int K, double alpha, const 
                        beta, kps, wk);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && ev && ev->end) e = hipEventRecord(ev->end, s);
-  if (e != hipSuccess || splits == 1) return e;
-  hipLaunchKernelGGL(k_splitk_reduce, dim3(1024), dim3(256), 0, s, M, N, splits, work, C, ldc, D, ldd, beta);
+  if (partials) *partials = splits;
+  if (e != hipSuccess || splits == 1 || partials) return e;
+  const GemmOutput o{C, ldc, D, ldd, beta};
+  hipLaunchKernelGGL(k_splitk_reduce, dim3(1024), dim3(256), 0, s, M, N, splits, work, o, o, N);
   return hipGetLastError();
 }
 
@@ -707,6 +736,154 @@ hipError_t launch_to_bf16_pairs(const float* x, long count, unsigned* out, hipSt
 hipError_t launch_to_bf16_pairs(const double* x, long count, unsigned* out, hipStream_t s) {
   if (count <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_to_bf16_pairs<double>, dim3(2048), dim3(256), 0, s, x, count, out);
+  return hipGetLastError();
+}
+
+namespace {
+constexpr int kOnsiteRows = 64;  // projector rows of one workgroup
+
+// Onsite products straight from the projection's split-K partials: P (the partials
+// of a column summed in split order) lives in LDS only, then per atom W(:, 0:m) =
+// D P and W(:, m:2m) = Q P, or with `shift` W(:, 0:m) = (D - shift_j Q) P in one
+// pass. Workgroup (g, j): atoms [group_atom[g], group_atom[g + 1]) (at most
+// kOnsiteRows rows, or one larger atom), column j. Bound: latency of the partials
+// (each read once). FP64 keeps the compensated scalar order of k_atom_blocks_comp.
+template <typename T>
+__global__ __launch_bounds__(256) void k_onsite_partials(int np, int columns, int splits,
+                                                         const double* __restrict__ partial,
+                                                         const int* __restrict__ group_atom,
+                                                         const int* __restrict__ atom_offset,
+                                                         const int* __restrict__ atom_rows,
+                                                         const long* __restrict__ block_offset,
+                                                         const double* __restrict__ dblk,
+                                                         const double* __restrict__ qblk,
+                                                         const double* __restrict__ shift, double* __restrict__ W,
+                                                         int which_mask) {
+#pragma clang fp contract(off)
+  extern __shared__ __attribute__((aligned(16))) unsigned char onsite_lds[];
+  double2* P = reinterpret_cast<double2*>(onsite_lds);
+  const int j = blockIdx.y, tid = threadIdx.x;
+  const int a0 = group_atom[blockIdx.x], a1 = group_atom[blockIdx.x + 1];
+  const int row0 = atom_offset[a0], rows = atom_offset[a1 - 1] + atom_rows[a1 - 1] - row0;
+  double2* sums = P + rows;  // three further quarters of the split sum
+  const long total = (long)np * columns;
+  const double2* src = reinterpret_cast<const double2*>(partial) + (long)j * np + row0;
+  // four threads a row: each sums a quarter of the splits in order
+  for (int e = tid; e < 4 * rows; e += 256) {
+    const int r = e % rows, q = e / rows;
+    const int s0 = splits * q / 4, s1 = splits * (q + 1) / 4;
+    double re = 0, im = 0;
+    int s = s0;
+    for (; s + 4 <= s1; s += 4) {
+      double2 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = src[(s + u) * total + r];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        re += v[u].x;
+        im += v[u].y;
+      }
+    }
+    for (; s < s1; ++s) {
+      const double2 v = src[s * total + r];
+      re += v.x;
+      im += v.y;
+    }
+    (q ? sums + (q - 1) * rows : P)[r] = double2{re, im};
+  }
+  __syncthreads();
+  for (int r = tid; r < rows; r += 256) {
+    double2 v = P[r];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      v.x += sums[q * rows + r].x;
+      v.y += sums[q * rows + r].y;
+    }
+    P[r] = v;
+  }
+  __syncthreads();
+  auto product = [&](const double* blk, int r, int i, const double2* p, double& re, double& im) {
+    if constexpr (sizeof(T) == 8) {
+      double rs = 0, rc = 0, is = 0, ic = 0;
+      auto add = [](double v, double& s, double& c) {
+        const double next = s + v;
+        const double back = next - s;
+        c += (s - (next - back)) + (v - back);
+        s = next;
+      };
+      auto term = [&](double x, double y, double& s, double& c) {
+        const double rounded = x * y;
+        add(rounded, s, c);
+        add(__builtin_fma(x, y, -rounded), s, c);
+      };
+      for (int k = 0; k < r; ++k) {
+        const double lr = blk[2 * (i + k * r)], li = blk[2 * (i + k * r) + 1];
+        term(lr, p[k].x, rs, rc);
+        term(-li, p[k].y, rs, rc);
+        term(lr, p[k].y, is, ic);
+        term(li, p[k].x, is, ic);
+      }
+      re = rs + rc;
+      im = is + ic;
+    } else {
+      float fr = 0.f, fi = 0.f;
+      for (int k = 0; k < r; ++k) {
+        const float lr = float(blk[2 * (i + k * r)]), li = float(blk[2 * (i + k * r) + 1]);
+        const float pr = float(p[k].x), pi = float(p[k].y);
+        fr += lr * pr - li * pi;
+        fi += lr * pi + li * pr;
+      }
+      re = fr;
+      im = fi;
+    }
+  };
+  double2* out = reinterpret_cast<double2*>(W) + (long)j * np + row0;
+  for (int e = tid; e < (shift ? 1 : 2) * rows; e += 256) {
+    const int row = e % rows, which = e / rows;
+    if (!shift && !((which_mask >> which) & 1)) continue;
+    int a = a0;
+    while (a + 1 < a1 && atom_offset[a + 1] - row0 <= row) ++a;
+    const int r = atom_rows[a], o = atom_offset[a] - row0;
+    const double2* p = P + o;
+    double re, im;
+    product((which ? qblk : dblk) + 2 * block_offset[a], r, row - o, p, re, im);
+    if (shift) {
+      double qr, qi;
+      product(qblk + 2 * block_offset[a], r, row - o, p, qr, qi);
+      re -= shift[j] * qr;
+      im -= shift[j] * qi;
+    }
+    out[(long)which * total + row] = double2{re, im};
+  }
+}
+}  // namespace
+
+std::vector<int> onsite_groups(const std::vector<int>& atom_rows) {
+  std::vector<int> first{0};
+  int rows = 0;
+  for (std::size_t a = 0; a < atom_rows.size(); ++a) {
+    if (rows && rows + atom_rows[a] > kOnsiteRows) {
+      first.push_back(int(a));
+      rows = 0;
+    }
+    rows += atom_rows[a];
+  }
+  first.push_back(int(atom_rows.size()));
+  return first;
+}
+
+hipError_t launch_onsite_partials(Precision prec, int np, int columns, int splits, const double* partial,
+                                  const int* group_atom, int groups, int group_rows, const int* atom_offset,
+                                  const int* atom_rows, const long* block_offset, const double* dblk,
+                                  const double* qblk, const double* shift, double* W, int which_mask, hipStream_t s) {
+  const std::size_t lds = 4 * std::size_t(group_rows) * 16;
+  if (columns > 65535 || group_rows > kOnsiteGroupRows) return hipErrorInvalidValue;
+  if (prec == Precision::FP64)
+    hipLaunchKernelGGL(k_onsite_partials<double>, dim3(groups, columns), dim3(256), lds, s, np, columns, splits,
+                       partial, group_atom, atom_offset, atom_rows, block_offset, dblk, qblk, shift, W, which_mask);
+  else
+    hipLaunchKernelGGL(k_onsite_partials<float>, dim3(groups, columns), dim3(256), lds, s, np, columns, splits,
+                       partial, group_atom, atom_offset, atom_rows, block_offset, dblk, qblk, shift, W, which_mask);
   return hipGetLastError();
 }
 

@@ -216,7 +216,8 @@ int max_lds_bytes() {
 
 template <typename T>
 hipError_t launch_local_h(const GridPlanDev& p, const double* x, long ldx, long columns, const double* kinetic,
-                          double* y, long ldy, void* t1, void* t2, hipStream_t stream) {
+                          double* y, long ldy, void* t1, void* t2, hipStream_t stream, const double* shift,
+                          double shift_scale) {
   if (columns <= 0) return hipSuccess;
   // one xy-plane per workgroup must fit the LDS of one workgroup
   if (plane_lds_bytes<T>(p.n0, p.n1) > size_t(max_lds_bytes())) return hipErrorInvalidConfiguration;
@@ -234,13 +235,13 @@ hipError_t launch_local_h(const GridPlanDev& p, const double* x, long ldx, long 
                        reinterpret_cast<const cx<T>*>(t1), reinterpret_cast<cx<T>*>(t2), p.stick_xy, p.nsticks, p.n0,
                        p.n1, p.n2, twx, twy, v, 0, p.xstart[0], p.xlines[0], p.xstart[1], p.xlines[1]);
   }
-  return launch_sticks_forward<T>(p, t2, columns, x, ldx, kinetic, y, ldy, stream);
+  return launch_sticks_forward<T>(p, t2, columns, x, ldx, kinetic, y, ldy, stream, shift, shift_scale);
 }
 
 template hipError_t launch_local_h<double>(const GridPlanDev&, const double*, long, long, const double*, double*, long,
-                                           void*, void*, hipStream_t);
+                                           void*, void*, hipStream_t, const double*, double);
 template hipError_t launch_local_h<float>(const GridPlanDev&, const double*, long, long, const double*, double*, long,
-                                          void*, void*, hipStream_t);
+                                          void*, void*, hipStream_t, const double*, double);
 
 hipError_t launch_column_scaled_add(const double* x, long ldx, double* y, long ldy, long rows, long columns,
                                     const double* theta, double scale, hipStream_t stream) {

@@ -24,11 +24,13 @@ struct GridPlanDev {
   long points = 0;  // plane waves
 };
 
-// y(:,c) = T x(:,c) + FFT_fwd(V . FFT_bwd(x(:,c))) / N for c < columns.
+// y(:,c) = T x(:,c) + FFT_fwd(V . FFT_bwd(x(:,c))) / N for c < columns, with
+// shift (columns values on the device) T - shift_scale shift[c] in the place of T.
 // t1/t2: stick buffers of columns * nsticks * n2 complex values of T.
 template <typename T>
 hipError_t launch_local_h(const GridPlanDev& p, const double* x, long ldx, long columns, const double* kinetic,
-                          double* y, long ldy, void* t1, void* t2, hipStream_t stream);
+                          double* y, long ldy, void* t1, void* t2, hipStream_t stream, const double* shift = nullptr,
+                          double shift_scale = 0);
 
 // y(:, j) += scale * theta[j] * x(:, j) for j < columns (theta on the device)
 hipError_t launch_column_scaled_add(const double* x, long ldx, double* y, long ldy, long rows, long columns,

@@ -30,12 +30,14 @@ hipError_t launch_plane_local(const GridPlanDev& p, const PlaneLocalPlan& plan, 
                               hipStream_t stream);
 
 // z-transforms of the sticks: x(:, c) gathered from the sphere into
-// t1[column][z slot][stick], and back with y = diag .* x + (transform) / count.
+// t1[column][z slot][stick], and back with y = diag .* x + (transform) / count
+// (diag - shift_scale shift[c] in the place of diag with a shift).
 template <typename T>
 hipError_t launch_sticks_backward(const GridPlanDev& p, const double* x, long ldx, long columns, void* t1,
                                   hipStream_t stream);
 template <typename T>
 hipError_t launch_sticks_forward(const GridPlanDev& p, const void* t2, long columns, const double* x, long ldx,
-                                 const double* diag, double* y, long ldy, hipStream_t stream);
+                                 const double* diag, double* y, long ldy, hipStream_t stream,
+                                 const double* shift = nullptr, double shift_scale = 0);
 
 }  // namespace sdft_hip

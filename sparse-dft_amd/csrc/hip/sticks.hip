@@ -95,7 +95,8 @@ __device__ __forceinline__ double divide(double a, double b, double inv) {
 template <int L1, int L2, typename T, bool HALF, int NT>
 __device__ __forceinline__ void forward(cx<T>* lines, const cx<T>* __restrict__ in, const int* __restrict__ stick_g,
                                         int nsticks, const cx<T>* __restrict__ tw, const double* __restrict__ x,
-                                        const double* __restrict__ diag, double* __restrict__ y, long n, double count) {
+                                        const double* __restrict__ diag, double* __restrict__ y, long n, double count,
+                                        double lower) {
   constexpr int S = sticks_of<L1, L2>(NT), L = L1 * L2, LS = L | 1;
   const int tid = threadIdx.x, first = blockIdx.x * S;
   if (first >= nsticks) return;
@@ -147,8 +148,9 @@ __device__ __forceinline__ void forward(cx<T>* lines, const cx<T>* __restrict__ 
 #pragma unroll
     for (int k = 0; k < L2; ++k)
       if (keeps<L2, HALF>(k)) {
-        const cx<double> r{d[k] * old[k].x + divide(double(v[k].x), count, inv),
-                           d[k] * old[k].y + divide(double(v[k].y), count, inv)};
+        const double t = d[k] - lower;
+        const cx<double> r{t * old[k].x + divide(double(v[k].x), count, inv),
+                           t * old[k].y + divide(double(v[k].y), count, inv)};
         ys.store(r, g[k] * 16);
       }
   }
@@ -177,16 +179,18 @@ __global__ __launch_bounds__(NT) void k_sticks_forward(const cx<T>* __restrict__
                                                        int nsticks, int n2, const cx<T>* __restrict__ tw,
                                                        const double* __restrict__ x, long ldx,
                                                        const double* __restrict__ diag, double* __restrict__ y,
-                                                       long ldy, long n, double count) {
+                                                       long ldy, long n, double count,
+                                                       const double* __restrict__ shift, double shift_scale) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   cx<T>* lines = reinterpret_cast<cx<T>*>(smem_raw);
   const long column = blockIdx.y;
   const cx<T>* in = t2 + column * (long)n2 * nsticks;
   const double* xc = x + 2 * column * ldx;
   double* yc = y + 2 * column * ldy;
+  const double lower = shift ? shift_scale * shift[column] : 0.0;
 #define SDFT_HIP_FORWARD(L, A, B) \
   case L:                         \
-    if constexpr (wide_split(A, B) == WIDE) forward<A, B, T, HALF, NT>(lines, in, stick_g, nsticks, tw, xc, diag, yc, n, count); \
+    if constexpr (wide_split(A, B) == WIDE) forward<A, B, T, HALF, NT>(lines, in, stick_g, nsticks, tw, xc, diag, yc, n, count, lower); \
     break;
   SDFT_HIP_LENGTH_SWITCH(n2, SDFT_HIP_FORWARD)
 #undef SDFT_HIP_FORWARD
@@ -247,14 +251,15 @@ hipError_t launch_sticks_backward(const GridPlanDev& p, const double* x, long ld
 
 template <typename T>
 hipError_t launch_sticks_forward(const GridPlanDev& p, const void* t2, long columns, const double* x, long ldx,
-                                 const double* diag, double* y, long ldy, hipStream_t stream) {
+                                 const double* diag, double* y, long ldy, hipStream_t stream, const double* shift,
+                                 double shift_scale) {
   const StickShape s = stick_shape<T>(p, columns);
   if (!s.grid.x || !s.lds) return hipErrorInvalidConfiguration;
   const cx<T>* tw = reinterpret_cast<const cx<T>*>(sizeof(T) == 8 ? p.tw64[2] : p.tw32[2]);
   for_shape(s, [&](auto wide, auto half, auto nt) {
     hipLaunchKernelGGL((k_sticks_forward<T, wide(), half(), nt()>), s.grid, dim3(nt()), s.lds, stream,
                        reinterpret_cast<const cx<T>*>(t2), p.stick_g, p.nsticks, p.n2, tw, x, ldx, diag, y, ldy,
-                       p.points, double(p.count));
+                       p.points, double(p.count), shift, shift_scale);
   });
   return hipGetLastError();
 }
@@ -262,9 +267,9 @@ hipError_t launch_sticks_forward(const GridPlanDev& p, const void* t2, long colu
 template hipError_t launch_sticks_backward<double>(const GridPlanDev&, const double*, long, long, void*, hipStream_t);
 template hipError_t launch_sticks_backward<float>(const GridPlanDev&, const double*, long, long, void*, hipStream_t);
 template hipError_t launch_sticks_forward<double>(const GridPlanDev&, const void*, long, const double*, long,
-                                                  const double*, double*, long, hipStream_t);
+                                                  const double*, double*, long, hipStream_t, const double*, double);
 template hipError_t launch_sticks_forward<float>(const GridPlanDev&, const void*, long, const double*, long,
-                                                 const double*, double*, long, hipStream_t);
+                                                 const double*, double*, long, hipStream_t, const double*, double);
 
 // Loads this file's code object on the calling thread (see module_prime.hpp).
 hipError_t prime_module_sticks() {

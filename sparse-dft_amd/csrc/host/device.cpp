@@ -220,9 +220,6 @@ Context::Context(int device) : device_(device) {
     throw std::runtime_error("HIP: rocblas_create_handle failed");
   }
   check(rocblas_set_stream(blas_, stream_), "rocblas_set_stream");
-  check(hipStreamCreateWithFlags(&aux_, hipStreamNonBlocking), "hipStreamCreate");
-  check(hipEventCreateWithFlags(&fork_event_, hipEventDisableTiming), "hipEventCreate");
-  check(hipEventCreateWithFlags(&join_event_, hipEventDisableTiming), "hipEventCreate");
 }
 
 PinnedStaging::PinnedStaging(std::size_t bytes) : cap_(bytes) {
@@ -295,28 +292,14 @@ void Context::download_bulk(void* host_dst, const void* device_src, std::size_t 
   }
 }
 
-void Context::fork() {
-  check(hipEventRecord(fork_event_, stream_), "fork record");
-  check(hipStreamWaitEvent(aux_, fork_event_, 0), "fork wait");
-}
-
-void Context::join() {
-  check(hipEventRecord(join_event_, aux_), "join record");
-  check(hipStreamWaitEvent(stream_, join_event_, 0), "join wait");
-}
-
 Context::~Context() {
-  if (aux_) (void)hipStreamSynchronize(aux_);
   (void)hipStreamSynchronize(stream_);
   for (hipEvent_t e : events_) (void)hipEventDestroy(e);
-  if (fork_event_) (void)hipEventDestroy(fork_event_);
-  if (join_event_) (void)hipEventDestroy(join_event_);
   for (int i = 0; i < 2; ++i) {
     if (bulk_[i]) (void)hipHostFree(bulk_[i]);
     if (bulk_done_[i]) (void)hipEventDestroy(bulk_done_[i]);
   }
   if (blas_) rocblas_destroy_handle(blas_);
-  if (aux_) (void)hipStreamDestroy(aux_);
   if (stream_) (void)hipStreamDestroy(stream_);
 }
 
@@ -346,7 +329,7 @@ void Context::clock_enable(bool on) {
   for (auto& c : clock_) c = ClockStat{};
 }
 
-LaunchEvents Context::clock_launch(int kind, double work, double bytes) {
+LaunchEvents Context::clock_launch(int kind, double work, double bytes, long products) {
   if (!clock_on_) return {};
   if (kind < 0 || kind >= kClockKinds) throw std::invalid_argument("HIP: invalid kernel clock kind");
   while (events_.size() < events_used_ + 2) {
@@ -354,7 +337,7 @@ LaunchEvents Context::clock_launch(int kind, double work, double bytes) {
     check(hipEventCreate(&e), "hipEventCreate");
     events_.push_back(e);
   }
-  pending_.push_back({kind, work, bytes, events_used_});
+  pending_.push_back({kind, work, bytes, products, events_used_});
   LaunchEvents ev{events_[events_used_], events_[events_used_ + 1]};
   events_used_ += 2;
   return ev;
@@ -367,7 +350,7 @@ Context::ClockStat Context::clock_stat(int kind) {
     float ms = 0.f;
     check(hipEventElapsedTime(&ms, events_[p.first_event], events_[p.first_event + 1]), "hipEventElapsedTime");
     auto& c = clock_[p.kind];
-    c.launches += 1;
+    c.launches += p.products;
     c.milliseconds += ms;
     c.work += p.work;
     c.bytes += p.bytes;
@@ -577,6 +560,7 @@ DeviceOperator::DeviceOperator(Context& ctx, const OperatorDesc& d) : ctx_(ctx) 
     atom_offset_.upload(offs.data(), offs.size(), s);
     atom_rows_.upload(rws.data(), rws.size(), s);
     atom_rows_host_ = rws;
+    upload_onsite_groups();
     block_offset_.upload(boffs.data(), boffs.size(), s);
     ctx_.sync();
   }
@@ -595,6 +579,19 @@ void DeviceOperator::set_chunk() {
     if (v > 0) cap = std::min<std::size_t>(cap, std::size_t(v));
   }
   chunk_ = std::max<std::size_t>(1, std::min<std::size_t>(cap, (std::size_t(512) << 20) / std::max<std::size_t>(1, per_col)));
+}
+
+void DeviceOperator::upload_onsite_groups() {
+  const std::vector<int> first = onsite_groups(atom_rows_host_);
+  onsite_groups_ = int(first.size()) - 1;
+  onsite_group_rows_ = 0;
+  for (int g = 0; g < onsite_groups_; ++g) {
+    int rows = 0;
+    for (int a = first[g]; a < first[g + 1]; ++a) rows += atom_rows_host_[a];
+    onsite_group_rows_ = std::max(onsite_group_rows_, rows);
+  }
+  onsite_group_.upload(first.data(), first.size(), ctx_.stream());
+  ctx_.sync();  // `first` ends here
 }
 
 // Columns of one pass over `columns`: passes of equal width (a narrow last pass
@@ -665,6 +662,7 @@ DeviceOperator::DeviceOperator(Context& ctx, const SnapshotArrays& sa) : ctx_(ct
       atom_offset_.upload(offs.data(), offs.size(), s);
       atom_rows_.upload(atom_rows_host_.data(), atom_rows_host_.size(), s);
       block_offset_.upload(boffs.data(), boffs.size(), s);
+      upload_onsite_groups();
     } else {
       const std::size_t cols = form_ == SnapshotArrays::Dense ? np_ : n_;
       if (sa.onsite_d.size() != np_ * cols || sa.onsite_q.size() != np_ * cols)
@@ -744,7 +742,7 @@ std::size_t DeviceOperator::device_bytes() const {
   std::size_t b = grid_.stick_g.bytes() + grid_.stick_xy.bytes() + grid_.stick_map.bytes();
   for (int a = 0; a < 3; ++a) b += grid_.tw64[a].bytes() + grid_.tw32[a].bytes();
   b += onsite_d_.bytes() + onsite_q_.bytes() + v64_.bytes() + kinetic_d_.bytes() + b64_.bytes() + dblk_.bytes() +
-       qblk_.bytes() + v32_.bytes() + b32_.bytes() + atom_offset_.bytes() + atom_rows_.bytes() + block_offset_.bytes() +
+       qblk_.bytes() + v32_.bytes() + b32_.bytes() + onsite_group_.bytes() + atom_offset_.bytes() + atom_rows_.bytes() + block_offset_.bytes() +
        t1_.bytes() + t2_.bytes() + p_.bytes() + w_.bytes();
   b += rs_w64_.bytes() + rs_sdiag_.bytes() + rs_w32_.bytes() + rs_woff_.bytes() + rs_poff_.bytes() +
        rs_points_.bytes() + rs_upoints_.bytes() + rs_estart_.bytes() + rs_eatom_.bytes() + rs_elocal_.bytes() +
@@ -834,6 +832,7 @@ DeviceOperator::StagingBytes DeviceOperator::staging_bytes(int which, long c, Pr
     z.work = zgemm_workspace_bytes(int(np), cc, int(n));
   }
   if (form_ != 3) z.work = std::max(z.work, zgemm_workspace_bytes(int(np), cc, int(form_ == 2 ? np : n)));
+  z.work = std::max(z.work, zgemm_workspace_bytes(int(n), which == 2 ? 2 * cc : cc, int(np)));
   z.work = std::max(z.work, zgemm_workspace_bytes(int(n), cc, int(np)));
   return z;
 }
@@ -1220,23 +1219,26 @@ void DeviceOperator::apply_chunk(int which, const double* x, long c, double* hy,
   hipStream_t s = ctx_.stream();
   const long n = long(n_), np = long(np_);
   const bool want_h = which != 1, want_s = which != 0;
-  // The local Hamiltonian (LDS/latency bound FFT pipeline) runs on the
-  // context's second stream beside the projector chain (MFMA GEMMs) on the
-  // main stream; the H back-projection adds to its output after the join.
-  const bool overlap = want_h && np;
+  // One stream: the local Hamiltonian beside the projector chain on a second one
+  // took longer at every size but the widest slab blocks (pair, us, two streams /
+  // one: 4 columns of 8 atoms 75 / 45, 40 of 16 atoms 109 / 96, 160 of 64 atoms FP64
+  // 1168 / 1157 and FP32 686 / 672; 160 of the slab 1304 / 1317): the events cost
+  // more than what the full kernels leave idle.
+  const bool f64 = prec == Precision::FP64;
   if (want_h) {
-    hipStream_t ls = overlap ? ctx_.aux_stream() : s;
-    if (overlap) ctx_.fork();
-    const bool f64 = prec == Precision::FP64;
     const double local_bytes = local_algorithmic_bytes(n, count_, c, f64);
     const LaunchEvents ev = ctx_.clock_launch(f64 ? Context::kLocalFP64 : Context::kLocalFP32, local_bytes, local_bytes);
-    if (ev.begin) check(hipEventRecord(ev.begin, ls), "hipEventRecord");
+    if (ev.begin) check(hipEventRecord(ev.begin, s), "hipEventRecord");
+    // (H - theta S) x: the identity part of S lowers T
+    const double lower = 1.0 + reg_;
     if (f64)
-      check(launch_local_h<double>(grid_.dev, x, n, c, kinetic_d_.p, hy, n, st.t1, st.t2, ls), "local H");
+      check(launch_local_h<double>(grid_.dev, x, n, c, kinetic_d_.p, hy, n, st.t1, st.t2, s, shift, lower), "local H");
     else
-      check(launch_local_h<float>(grid_.dev, x, n, c, kinetic_d_.p, hy, n, st.t1, st.t2, ls), "local H");
-    if (ev.end) check(hipEventRecord(ev.end, ls), "hipEventRecord");
+      check(launch_local_h<float>(grid_.dev, x, n, c, kinetic_d_.p, hy, n, st.t1, st.t2, s, shift, lower), "local H");
+    if (ev.end) check(hipEventRecord(ev.end, s), "hipEventRecord");
   }
+  const int kind = f64 ? Context::kGemmFP64 : bf16 ? Context::kGemmBF16 : Context::kGemmFP32;
+  const int b_bytes = f64 ? 16 : bf16 ? 4 : 8;
   auto gemm = [&](int aop, long M, long K, double alpha, const double* A, long lda, const double* B, long ldb,
                   double* C, long ldc, const double* D, long ldd, double beta) {
     ctx_.zgemm_into(prec, aop, 0, M, c, K, alpha, A, lda, B, ldb, C, ldc, D, ldd, beta, st.work, st.work_bytes);
@@ -1250,63 +1252,75 @@ void DeviceOperator::apply_chunk(int which, const double* x, long c, double* hy,
     const long inner = dense ? np : n, ldr = dense ? np : n;
     if (want_h) gemm(0, np, inner, 1.0, onsite_d_.p, np, rhs, ldr, st.w, np, nullptr, 0, 0.0);
     if (want_s) gemm(0, np, inner, 1.0, onsite_q_.p, np, rhs, ldr, st.w + 2 * np * c, np, nullptr, 0, 0.0);
+    if (shift) check(launch_column_scaled_add(st.w + 2 * np * c, np, st.w, np, np, c, shift, -1.0, s), "onsite shift");
   } else if (np) {
-    if (prec == Precision::FP64)
-      gemm(0, np, n, 1.0, b64_.p, np, x, n, st.p, np, nullptr, 0, 0.0);
-    else if (bf16) {
-      const LaunchEvents ev =
-          ctx_.clock_launch(Context::kGemmBF16, 8.0 * np * c * n, gemm_algorithmic_bytes(np, c, n, 4, false));
+    // the projection is left as split-K partials, which the onsite kernel sums
+    const bool direct = onsite_group_rows_ <= kOnsiteGroupRows;
+    int partials = 1;
+    int* const left = direct ? &partials : nullptr;
+    const LaunchEvents ev = ctx_.clock_launch(kind, 8.0 * np * c * n, gemm_algorithmic_bytes(np, c, n, b_bytes, false));
+    if (f64)
+      check(zgemm(prec, 0, 0, int(np), int(c), int(n), 1.0, b64_.p, np, x, n, st.p, np, nullptr, 0, 0.0, st.work,
+                  st.work_bytes, s, &ev, left),
+            "projection");
+    else if (bf16)
       check(zgemm_bf16_storage(0, int(np), int(c), int(n), 1.0, projectors_bf16(), np, x, n, st.p, np, nullptr, 0, 0.0,
-                               st.work, st.work_bytes, s, &ev),
+                               st.work, st.work_bytes, s, &ev, left),
             "projection");
-    } else {
-      const LaunchEvents ev =
-          ctx_.clock_launch(Context::kGemmFP32, 8.0 * np * c * n, gemm_algorithmic_bytes(np, c, n, 8, false));
+    else
       check(zgemm_f32_storage(0, 0, int(np), int(c), int(n), 1.0, b32_.p, np, x, n, st.p, np, nullptr, 0, 0.0, st.work,
-                              st.work_bytes, s, &ev),
+                              st.work_bytes, s, &ev, left),
             "projection");
-    }
     const int mask = (want_h ? 1 : 0) | (want_s ? 2 : 0);
-    check(launch_atom_blocks(prec, int(np), int(c), atoms_, atom_offset_.p, atom_rows_.p, block_offset_.p, dblk_.p,
-                             qblk_.p, st.p, np, st.w, np, mask, s),
-          "onsite blocks");
-  }
-  auto backproject = [&](const double* w, double* out, const double* d, double beta) {
-    if (prec == Precision::FP64)
-      gemm(1, n, np, 1.0, b64_.p, np, w, np, out, n, d, n, beta);
-    else if (bf16) {
-      const LaunchEvents ev =
-          ctx_.clock_launch(Context::kGemmBF16, 8.0 * n * c * np, gemm_algorithmic_bytes(n, c, np, 4, beta != 0.0));
-      check(zgemm_bf16_storage(1, int(n), int(c), int(np), 1.0, projectors_bf16(), np, w, np, out, n, d, n, beta,
-                               st.work, st.work_bytes, s, &ev),
-            "back projection");
+    if (direct) {
+      check(launch_onsite_partials(prec, int(np), int(c), partials, partials > 1 ? st.work : st.p, onsite_group_.p,
+                                   onsite_groups_, onsite_group_rows_, atom_offset_.p, atom_rows_.p, block_offset_.p,
+                                   dblk_.p, qblk_.p, shift, st.w, mask, s),
+            "onsite blocks");
     } else {
-      const LaunchEvents ev =
-          ctx_.clock_launch(Context::kGemmFP32, 8.0 * n * c * np, gemm_algorithmic_bytes(n, c, np, 8, beta != 0.0));
-      check(zgemm_f32_storage(1, 0, int(n), int(c), int(np), 1.0, b32_.p, np, w, np, out, n, d, n, beta, st.work,
-                              st.work_bytes, s, &ev),
-            "back projection");
+      // an atom with more projectors than a workgroup sums in LDS
+      check(launch_atom_blocks(prec, int(np), int(c), atoms_, atom_offset_.p, atom_rows_.p, block_offset_.p, dblk_.p,
+                               qblk_.p, st.p, np, st.w, np, mask, s),
+            "onsite blocks");
+      if (shift) check(launch_column_scaled_add(st.w + 2 * np * c, np, st.w, np, np, c, shift, -1.0, s), "onsite shift");
     }
-  };
-  if (shift) {
-    // (H - theta S) x = local H x + B^H (D - theta Q) P - theta (1 + reg) x
-    if (np) {
-      check(launch_column_scaled_add(st.w + 2 * np * c, np, st.w, np, np, c, shift, -1.0, s), "onsite shift");
-      if (overlap) ctx_.join();
-      backproject(st.w, hy, hy, 1.0);
-    }
-    check(launch_column_scaled_add(x, n, hy, n, n, c, shift, -(1.0 + reg_), s), "identity shift");
+  }
+  if (!np) {
+    if (want_s && !shift) check(launch_scale_copy(x, n, sy, n, n, c, 1.0 + reg_, s), "overlap identity");
     return;
   }
-  if (np) {
-    if (want_s) backproject(st.w + 2 * np * c, sy, x, 1.0 + reg_);
-    if (want_h) {
-      if (overlap) ctx_.join();
-      backproject(st.w, hy, hy, 1.0);
-    }
-  } else if (want_s) {
-    check(launch_scale_copy(x, n, sy, n, n, c, 1.0 + reg_, s), "overlap identity");
+  const GemmOutput h{hy, n, hy, n, 1.0}, sx{sy, n, x, n, 1.0 + reg_};
+  const bool pair = want_h && want_s && !shift;
+  const long columns = pair ? 2 * c : c;
+  const LaunchEvents ev =
+      ctx_.clock_launch(kind, 8.0 * n * columns * np, gemm_algorithmic_bytes(n, columns, np, b_bytes, true),
+                        pair ? 2 : 1);
+  if (pair) {
+    // H and S in one product over the projectors: W holds (D P | Q P)
+    if (f64)
+      check(zgemm_two_outputs(1, int(n), int(c), int(c), int(np), b64_.p, np, st.w, np, h, sx, st.work, st.work_bytes, s,
+                              &ev),
+            "back projection");
+    else
+      check(zgemm_two_outputs(1, int(n), int(c), int(c), int(np), b32_.p, np, st.w, np, h, sx, st.work, st.work_bytes, s,
+                              &ev),
+            "back projection");
+    return;
   }
+  const GemmOutput& o = want_h ? h : sx;
+  const double* w = want_h ? st.w : st.w + 2 * np * c;
+  if (f64)
+    check(zgemm(prec, 1, 0, int(n), int(c), int(np), 1.0, b64_.p, np, w, np, o.C, o.ldc, o.D, o.ldd, o.beta, st.work,
+                st.work_bytes, s, &ev),
+          "back projection");
+  else if (bf16)
+    check(zgemm_bf16_storage(1, int(n), int(c), int(np), 1.0, projectors_bf16(), np, w, np, o.C, o.ldc, o.D, o.ldd, o.beta,
+                             st.work, st.work_bytes, s, &ev),
+          "back projection");
+  else
+    check(zgemm_f32_storage(1, 0, int(n), int(c), int(np), 1.0, b32_.p, np, w, np, o.C, o.ldc, o.D, o.ldd, o.beta, st.work,
+                            st.work_bytes, s, &ev),
+          "back projection");
 }
 
 }  // namespace sdft_hip

@@ -108,11 +108,6 @@ class Context {
   ~Context();
   int device() const { return device_; }
   hipStream_t stream() const { return stream_; }
-  // Second stream of the context (default priority) for work that overlaps the
-  // main stream inside one operation: fork() makes it wait for everything
-  // queued on the main stream so far, join() makes the main stream wait for
-  // everything queued on it.
-  hipStream_t aux_stream() const { return aux_; }
   // pinned staging of the main stream's control transfers (allocated once)
   PinnedStaging& staging();
   // bulk transfers between pageable host memory and the device on the main
@@ -120,8 +115,6 @@ class Context {
   // copy of the other. Both return with the transfer complete.
   void upload_bulk(void* device_dst, const void* host_src, std::size_t bytes);
   void download_bulk(void* host_dst, const void* device_src, std::size_t bytes);
-  void fork();
-  void join();
   rocblas_handle blas() const { return blas_; }
   const std::string& name() const { return name_; }
   void sync() { check(hipStreamSynchronize(stream_), "hipStreamSynchronize"); }
@@ -161,7 +154,8 @@ class Context {
   };
   void clock_enable(bool on);  // clears the sums either way
   // Events to record for one launch (both null when the clock is off).
-  LaunchEvents clock_launch(int kind, double work, double bytes);
+  // `products`: how many GEMMs (or local-H pipelines) the launch stands for.
+  LaunchEvents clock_launch(int kind, double work, double bytes, long products = 1);
   ClockStat clock_stat(int kind);  // synchronises the stream and folds pending pairs
 
   // caches for the drop-in host-pointer entry points (identity tokens)
@@ -190,8 +184,6 @@ class Context {
  private:
   int device_;
   hipStream_t stream_{};
-  hipStream_t aux_{};
-  hipEvent_t fork_event_{}, join_event_{};
   std::unique_ptr<PinnedStaging> staging_;
   char* bulk_[2] = {nullptr, nullptr};
   hipEvent_t bulk_done_[2] = {};
@@ -206,6 +198,7 @@ class Context {
   struct PendingLaunch {
     int kind;
     double work, bytes;
+    long products;
     std::size_t first_event;
   };
   std::vector<PendingLaunch> pending_;
@@ -369,7 +362,9 @@ class DeviceOperator {
   DevBuf<double> v64_, kinetic_d_, b64_, dblk_, qblk_;
   DevBuf<float> v32_, b32_;
   DevBuf<unsigned> b16_;
-  DevBuf<int> atom_offset_, atom_rows_;
+  DevBuf<int> atom_offset_, atom_rows_, onsite_group_;
+  int onsite_groups_ = 0, onsite_group_rows_ = 0;
+  void upload_onsite_groups();
   DevBuf<long> block_offset_;
   int atoms_ = 0;
   DevBuf<char> t1_, t2_;

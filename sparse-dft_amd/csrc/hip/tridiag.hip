@@ -1,31 +1,32 @@
 // Householder reduction of a Hermitian matrix to real symmetric tridiagonal
-// form in one cooperative launch (the Rayleigh-Ritz eigensolve of the block
-// Davidson). Output follows LAPACK zhetrd with uplo = 'L' (d, e, tau and the
-// reflector tails v(k+2:n) in column k), so that a tridiagonal eigensolver and
-// zunmtr complete the decomposition.
+// form in one launch (the Rayleigh-Ritz eigensolve of the block Davidson). Output
+// follows LAPACK zhetrd with uplo = 'L' (d, e, tau and the reflector tails
+// v(k+2:n) in column k), so that a tridiagonal eigensolver and zunmtr complete the
+// decomposition.
 //
 // Layout: every workgroup keeps the rows g, g + G, g + 2G, ... of the matrix in
 // LDS for the whole reduction (the matrix never returns to HBM). Step k starts
-// with reflector k formed and p_i = sum_j A_ij v_j staged for the own rows,
+// with reflector k formed and p_i = sum_j A_ij v_j of every row i > k published
 // together with the pre-update A_{i,k+1}:
-//   1. publication of the staged values and one grid barrier;
-//   2. every workgroup loads all published values at once and reduces
-//      (tau p)^H v;
-//   3. w = tau p - (tau/2)(tau p)^H v v (in registers), the next column for all
-//      rows from the published A_{i,k+1}, the rank-2 update of the own rows;
-//   4. reflector k + 1 from the new column, formed redundantly by every
-//      workgroup (identical code and data, so identical bits everywhere), and
-//      the products of step k + 1 on the updated rows.
-// The published vectors are double-buffered by step parity, so one barrier per
-// column suffices. Each workgroup raises its own arrival flag (one cache line
-// per workgroup, no read-modify-write contention) and polls all flags with one
-// wave, with a bounded wait: on expiry it raises an abort flag that every
-// workgroup observes, and all workgroups leave the kernel.
-// Every published value is stored and loaded with agent-scope relaxed atomics
-// (sc1 accesses, coherent across the XCDs' L2 caches); a workgroup raises its
-// flag only after its stores have completed (vmcnt(0)), and readers load the
-// values only after they have seen every flag. This needs no L2 write-back or
-// invalidate, which an agent-scope fence would issue on every column.
+//   1. every thread polls the published values of its entries until all have
+//      arrived and reduces (tau p)^H v over the workgroup;
+//   2. w = tau p - (tau/2)(tau p)^H v v (in registers), the next column for all
+//      rows from the published A_{i,k+1}, the rank-2 update of the own rows and
+//      |column tail|^2 over the workgroup;
+//   3. reflector k + 1 from the new column, formed redundantly by every workgroup
+//      (identical code and data, so identical bits everywhere), and the products of
+//      step k + 1 on the updated rows with the unscaled column (the scale follows),
+//      each published by the wave that formed it.
+// The exchange is one memory round trip a column: the values themselves say that
+// they have arrived. A word not yet published is all ones (a NaN that is never
+// published); three buffers take turns, and a workgroup refills its own
+// entries of the one that every other has left, completed before its next
+// publication. A workgroup without rows left leaves the kernel, so that whoever
+// still reads a step has published the step before. Waits are bounded: on expiry an
+// abort flag ends every workgroup.
+// Every published word is stored and loaded with agent-scope relaxed atomics
+// (sc1 accesses, coherent across the XCDs' L2 caches), which needs no L2 write-back
+// or invalidate (an agent-scope fence would issue one on every column).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -40,7 +41,9 @@ namespace {
 constexpr int kThreads = 512;
 constexpr int kWaves = kThreads / 64;
 constexpr long kSpinLimit = 1L << 20;
-constexpr int kPerThread = (kHetrdMaxOrder + kThreads - 1) / kThreads;  // trailing entries per thread
+constexpr unsigned long long kMissing = ~0ull;  // a published word that has not arrived
+constexpr int kBuffers = 3;
+constexpr int kWords = 4;  // of one published row: p_i, A_{i,k+1}
 
 // Aligned to 16 bytes: one element is one 128-bit LDS access (the dynamic LDS
 // base is declared 16-byte aligned below, past the static variables).
@@ -55,254 +58,236 @@ __device__ inline Z zscale(Z a, double s) { return {a.x * s, a.y * s}; }
 
 __device__ inline double wave_sum(double v) { return wave::sum(v); }
 
-// Sum of one double over the workgroup in a fixed order; every thread gets it.
-__device__ double block_sum(double v, double* scratch) {
-  v = wave_sum(v);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  __syncthreads();
-  if (lane == 0) scratch[wave] = v;
-  __syncthreads();
-  double t = 0.;
+__device__ inline void publish(unsigned long long* slot, Z p, Z c) {
+  const double v[kWords] = {p.x, p.y, c.x, c.y};
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) t += scratch[w];
-  return t;
+  for (int w = 0; w < kWords; ++w) {
+    unsigned long long bits = __builtin_bit_cast(unsigned long long, v[w]);
+    if (bits == kMissing) bits = 0x7FF8000000000000ull;  // an input's NaN of all ones becomes the plain one
+    __hip_atomic_store(slot + w, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 }
 
-__device__ Z block_zsum(Z v, double* scratch) {
-  v.x = wave_sum(v.x);
-  v.y = wave_sum(v.y);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  __syncthreads();
-  if (lane == 0) {
-    scratch[2 * wave] = v.x;
-    scratch[2 * wave + 1] = v.y;
-  }
-  __syncthreads();
-  Z t{0., 0.};
+// Polls one row's words until all have arrived; false when the wait expired or
+// another workgroup gave up.
+__device__ bool receive(const unsigned long long* slot, int* abort_flag, Z& p, Z& c) {
+  unsigned long long w[kWords];
+  for (long spin = 0;; ++spin) {
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    t.x += scratch[2 * w];
-    t.y += scratch[2 * w + 1];
+    for (int u = 0; u < kWords; ++u)
+      w[u] = __hip_atomic_load(slot + u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (w[0] != kMissing && w[1] != kMissing && w[2] != kMissing && w[3] != kMissing) break;
+    if ((spin & 15) == 15 &&
+        __hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != kHetrdRunning)
+      return false;
+    if (spin > kSpinLimit) {
+      __hip_atomic_store(abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return false;
+    }
   }
-  return t;
+  p = {__builtin_bit_cast(double, w[0]), __builtin_bit_cast(double, w[1])};
+  c = {__builtin_bit_cast(double, w[2]), __builtin_bit_cast(double, w[3])};
+  return true;
 }
 
-__device__ inline void store_published(Z* p, Z v) {
-  double* q = reinterpret_cast<double*>(p);
-  __hip_atomic_store(q, v.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(q + 1, v.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline Z load_published(const Z* p) {
-  const double* q = reinterpret_cast<const double*>(p);
-  return {__hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
-          __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)};
-}
 // s_waitcnt vmcnt(0) with the other counters unconstrained (gfx9 encoding)
 constexpr int kWaitStores = 0x0F70;
 
-// Grid barrier with publication: the workgroup's staged values (count entries
-// of `src`, LDS, to dst[index[j]]) are stored by as many threads, each waits
-// for its stores to complete, and thread 0 raises the workgroup's arrival flag
-// to `step` (one flag per workgroup, each on its own 64-byte line, so arrivals
-// never contend). Thread q then polls the flag of workgroup q (every flag is
-// watched at once, so the wait ends one memory round trip after the last
-// arrival). Returns false when the wait expired or another workgroup gave up.
-constexpr int kFlagStride = 16;  // unsigned ints per flag line
-__device__ bool publish_and_wait(unsigned* flags, int* abort_flag, unsigned step, int count, const int* index,
-                                 const Z* src_p, const Z* src_c, Z* dst_p, Z* dst_c) {
-  __syncthreads();
-  const int tid = threadIdx.x;
-  for (int j = tid; j < count; j += kThreads) {
-    store_published(dst_p + index[j], src_p[j]);
-    store_published(dst_c + index[j], src_c[j]);
+// LDS of one workgroup: rpw matrix rows, the current column, the current
+// reflector, the staged products of the own rows, wave partials of two sums.
+struct HetrdLds {
+  Z *rows, *col, *v, *staged, *dot;
+  double* norm;
+  __device__ HetrdLds(double* base, int n, int rpw) {
+    rows = reinterpret_cast<Z*>(base);
+    col = rows + size_t(rpw) * n;
+    v = col + n;
+    staged = v + n;
+    dot = staged + rpw;
+    norm = reinterpret_cast<double*>(dot + kWaves);
   }
-  __builtin_amdgcn_s_waitcnt(kWaitStores);
-  __syncthreads();
-  if (tid == 0)
-    __hip_atomic_store(flags + blockIdx.x * kFlagStride, step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  int ok = 1;
-  for (int q = tid; q < int(gridDim.x) && ok; q += kThreads) {
-    for (long spin = 0;; ++spin) {
-      if (__hip_atomic_load(flags + q * kFlagStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= step) break;
-      if (__hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-        ok = 0;
-        break;
-      }
-      if (spin > kSpinLimit) {
-        __hip_atomic_fetch_or(abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        ok = 0;
-        break;
-      }
-      __builtin_amdgcn_s_sleep(1);
-    }
-  }
-  return __syncthreads_and(ok) != 0;
+};
+size_t lds_bytes(int n, int rpw) {
+  return (size_t(rpw) * n + 2 * size_t(n) + size_t(rpw) + kWaves) * sizeof(Z) + kWaves * sizeof(double);
 }
 
-// Reflector of the column held in `col` at rows c0 + 1 .. n - 1 (LAPACK zlarfg
-// conventions, m = n - c0 - 1 entries): writes v[0..m) (v[0] = 1) and, for
-// workgroup 0, d[c0], e[c0], tau[c0] and the reflector tail. `xn2` is the sum
-// of |col[j]|^2 over j >= c0 + 2. Returns tau. Ends with a block barrier.
-__device__ Z form_reflector(const Z* col, int c0, int n, double xn2, Z* v, Z* __restrict__ refl, long ldr,
-                            double* __restrict__ d, double* __restrict__ e, Z* __restrict__ tau) {
-  const int tid = threadIdx.x, m = n - c0 - 1;
-  const Z alpha = col[c0 + 1];
-  Z t{0., 0.}, scale{0., 0.};
-  double beta;
-  if (xn2 == 0. && alpha.y == 0.) {
-    // column already reduced: H = I - 2 e1 e1^T (beta = -alpha) instead of
-    // LAPACK's tau = 0; rocSOLVER zunmtr returned NaN columns for reflector
-    // sets with tau = 0 at orders of a few hundred (real tridiagonal inputs)
-    beta = -alpha.x;
-    t = {2., 0.};
-  } else {
-    const double nrm = sqrt(alpha.x * alpha.x + alpha.y * alpha.y + xn2);
-    beta = alpha.x >= 0. ? -nrm : nrm;
-    t = {(beta - alpha.x) / beta, -alpha.y / beta};
-    const Z den{alpha.x - beta, alpha.y};  // 1 / (alpha - beta)
-    const double dd = den.x * den.x + den.y * den.y;
-    scale = {den.x / dd, -den.y / dd};
-  }
-  for (int j = tid; j < m; j += kThreads) v[j] = j == 0 ? Z{1., 0.} : zmul(col[c0 + 1 + j], scale);
-  if (blockIdx.x == 0) {
-    if (tid == 0) {
-      d[c0] = col[c0].x;
-      e[c0] = beta;
-      tau[c0] = t;
-    }
-    for (int j = 2 + tid; j <= m; j += kThreads) refl[(c0 + j) + size_t(c0) * ldr] = zmul(col[c0 + j], scale);
-  }
-  __syncthreads();
-  return t;
-}
-
-// p_i = sum_j A_ij v_j over the trailing columns c0 + 1 .. n - 1 for the own
-// rows i > c0 (one wave per row), staged in LDS with A_{i,c0+1}; returns the
-// number of staged rows through `staged`. Ends with a block barrier.
-__device__ void stage_products(const Z* rows, int n, int rpw, int c0, const Z* v, Z* stage_p, Z* stage_c,
-                               int* stage_i, int* staged) {
-  const int tid = threadIdx.x, lane = tid & 63, g = blockIdx.x, G = gridDim.x, m = n - c0 - 1;
-  const int first = c0 + 1 - g <= 0 ? 0 : (c0 + 1 - g + G - 1) / G;
-  for (int r = first + (tid >> 6); r < rpw; r += kWaves) {
-    const int i = g + r * G;
-    if (i >= n) break;
-    const Z* row = rows + size_t(r) * n + (c0 + 1);
-    Z acc{0., 0.};
-    for (int j = lane; j < m; j += 64) acc = zadd(acc, zmul(row[j], v[j]));
-    acc.x = wave_sum(acc.x);
-    acc.y = wave_sum(acc.y);
-    if (lane == 0) {
-      stage_p[r - first] = acc;
-      stage_c[r - first] = row[0];
-      stage_i[r - first] = i;
-    }
-  }
-  if (tid == 0) {
-    int cnt = 0;
-    for (int r = first; r < rpw && g + r * G < n; ++r) ++cnt;
-    *staged = cnt;
-  }
-  __syncthreads();
-}
-
+// KP entries of a column per thread (n <= KP * kThreads).
+template <int KP>
 __global__ __launch_bounds__(kThreads) void k_hetrd_lds(const Z* __restrict__ a, long lda, int n, int rpw,
                                                         Z* __restrict__ refl, long ldr, double* __restrict__ d,
                                                         double* __restrict__ e, Z* __restrict__ tau,
-                                                        Z* __restrict__ pub_p, Z* __restrict__ pub_c,
-                                                        unsigned* __restrict__ flags, int* __restrict__ abort_flag) {
+                                                        unsigned long long* __restrict__ pub,
+                                                        int* __restrict__ abort_flag) {
   extern __shared__ __attribute__((aligned(16))) double lds_raw[];
-  Z* rows = reinterpret_cast<Z*>(lds_raw);  // rpw x n
-  Z* vbuf = rows + size_t(rpw) * n;         // two reflectors (steps of both parities), n each
-  Z* col = vbuf + 2 * size_t(n);            // current column, n
-  double* scratch = reinterpret_cast<double*>(col + n);  // 2 * kWaves
-  Z* stage_p = reinterpret_cast<Z*>(scratch + 2 * kWaves);  // rpw staged p_i
-  Z* stage_c = stage_p + rpw;                               // rpw staged A_{i,k+1}
-  int* stage_i = reinterpret_cast<int*>(stage_c + rpw);     // rpw row indices
-  __shared__ int staged;
+  __shared__ int expired;
+  __shared__ Z first_p;  // tau p of the first row
+  const HetrdLds lds(lds_raw, n, rpw);
+  const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int out = (n - 1) % G;  // the workgroup of the last row writes d, e, tau and the reflectors
+  auto slot = [&](int step, int row) { return pub + kWords * (size_t(step % kBuffers) * n + row); };
+  auto first_row = [&](int i0) { return i0 <= g ? 0 : (i0 - g + G - 1) / G; };  // first r with g + r G >= i0
 
-  const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x;
+  // Reflector of the column in lds.col at rows c0 + 1 .. n - 1 (LAPACK zlarfg
+  // conventions; |tail|^2 as wave partials in lds.norm, the workgroup's barrier
+  // passed), this thread's entries of it in vj and its copy in lds.v, the outputs,
+  // and the products of the own rows, published for step c0. Returns tau.
+  auto reflect = [&](int c0, Z (&vj)[KP]) {
+    const int m = n - c0 - 1;
+    const Z* col = lds.col;
+    double xn2 = 0.;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) xn2 += lds.norm[w];
+    const Z alpha = col[1];
+    Z t{0., 0.}, scale{0., 0.};
+    double beta;
+    if (xn2 == 0. && alpha.y == 0.) {
+      // column already reduced: H = I - 2 e1 e1^T (beta = -alpha) instead of
+      // LAPACK's tau = 0; rocSOLVER zunmtr returned NaN columns for reflector
+      // sets with tau = 0 at orders of a few hundred (real tridiagonal inputs)
+      beta = -alpha.x;
+      t = {2., 0.};
+    } else {
+      const double nrm = sqrt(alpha.x * alpha.x + alpha.y * alpha.y + xn2);
+      beta = alpha.x >= 0. ? -nrm : nrm;
+      t = {(beta - alpha.x) / beta, -alpha.y / beta};
+      const Z den{alpha.x - beta, alpha.y};  // 1 / (alpha - beta)
+      const double dd = den.x * den.x + den.y * den.y;
+      scale = {den.x / dd, -den.y / dd};
+    }
+    // one wave a row: sum_j A_ij col_j over the tail, scaled, plus A_{i,c0+1} (v = 1)
+    for (int r = first_row(c0 + 1) + wave; r < rpw; r += kWaves) {
+      const int i = g + r * G;
+      if (i >= n) break;
+      const Z* row = lds.rows + size_t(r) * n + c0;
+      Z acc{0., 0.};
+      for (int j = 2 + lane; j <= m; j += 64) acc = zadd(acc, zmul(row[j], col[j]));
+      acc.x = wave_sum(acc.x);
+      acc.y = wave_sum(acc.y);
+      if (lane == 0) {
+        const Z head = row[1], p = zadd(head, zmul(scale, acc));
+        publish(slot(c0, i), p, head);
+        lds.staged[r] = p;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < KP; ++q) {
+      const int j = tid + q * kThreads;
+      if (j < m) {
+        vj[q] = j == 0 ? Z{1., 0.} : zmul(col[1 + j], scale);
+        lds.v[j] = vj[q];
+        if (g == out && j > 0) refl[(c0 + 1 + j) + size_t(c0) * ldr] = vj[q];
+      }
+    }
+    if (g == out && tid == 0) {
+      d[c0] = col[0].x;
+      e[c0] = beta;
+      tau[c0] = t;
+    }
+    return t;
+  };
+  // |tail|^2 of the thread's entries of the column at c0 (entry j at row c0 + j) into
+  // the wave partials, the entries into lds.col
+  auto column = [&](const Z (&cv)[KP], int length) {
+    double part = 0.;
+#pragma unroll
+    for (int q = 0; q < KP; ++q) {
+      const int j = tid + q * kThreads;
+      if (j < length) {
+        lds.col[j] = cv[q];
+        if (j >= 2) part += cv[q].x * cv[q].x + cv[q].y * cv[q].y;
+      }
+    }
+    part = wave_sum(part);
+    if (lane == 0) lds.norm[wave] = part;
+  };
+
   // row i of the Hermitian input is the conjugate of column i (coalesced read)
   for (int r = 0; r < rpw; ++r) {
     const int i = g + r * G;
     if (i >= n) break;
-    for (int j = tid; j < n; j += kThreads) rows[size_t(r) * n + j] = zconj(a[j + size_t(i) * lda]);
+    for (int j = tid; j < n; j += kThreads) lds.rows[size_t(r) * n + j] = zconj(a[j + size_t(i) * lda]);
   }
-  for (int j = tid; j < n; j += kThreads) col[j] = a[j];
-  __syncthreads();
-  // prologue: reflector 0 and the products of step 0
-  Z t;
-  {
-    double part = 0.;
-    for (int j = 2 + tid; j < n; j += kThreads) part += col[j].x * col[j].x + col[j].y * col[j].y;
-    const double xn2 = block_sum(part, scratch);
-    t = form_reflector(col, 0, n, xn2, vbuf, refl, ldr, d, e, tau);
-    stage_products(rows, n, rpw, 0, vbuf, stage_p, stage_c, stage_i, &staged);
-  }
-  for (int k = 0; k + 1 < n; ++k) {
-    const int m = n - k - 1;  // order of the trailing block
-    Z* v = vbuf + size_t(k & 1) * n;
-    Z* vn = vbuf + size_t((k + 1) & 1) * n;
-    Z* pp = pub_p + size_t(k & 1) * n;
-    Z* pc = pub_c + size_t(k & 1) * n;
-    const int first = k + 1 - g <= 0 ? 0 : (k + 1 - g + G - 1) / G;
-    // ---- 1. publication and grid barrier
-    if (!publish_and_wait(flags, abort_flag, unsigned(k + 1), staged, stage_i, stage_p, stage_c, pp, pc)) return;
-    // ---- 2. all loads issued at once (one round trip); partial (tau p)^H v
-    Z pw[kPerThread], pcv[kPerThread];
-    const Z p0 = load_published(pp + k + 1);
+  Z cv[KP], vj[KP];
 #pragma unroll
-    for (int q = 0; q < kPerThread; ++q) {
-      const int j = tid + q * kThreads;
-      if (j < m) {
-        pw[q] = load_published(pp + k + 1 + j);
-        pcv[q] = load_published(pc + k + 1 + j);
-      }
-    }
+  for (int q = 0; q < KP; ++q) {
+    const int j = tid + q * kThreads;
+    cv[q] = j < n ? a[j] : Z{0., 0.};
+  }
+  if (tid == 0) expired = 0;
+  column(cv, n);
+  __syncthreads();
+  Z t = reflect(0, vj);
+  for (int k = 0; k + 1 < n; ++k) {
+    const int m = n - k - 1, first = first_row(k + 1);
+    if (first >= rpw || g + first * G >= n) return;  // no row left (the last row's workgroup stays)
+    // ---- 1. the published products of every row; partial (tau p)^H v
+    Z p[KP], c[KP];
+    bool ok = true;
     Z dot{0., 0.};
 #pragma unroll
-    for (int q = 0; q < kPerThread; ++q) {
-      const int j = tid + q * kThreads;
-      if (j < m) dot = zadd(dot, zmul(zconj(zmul(t, pw[q])), v[j]));
-    }
-    dot = block_zsum(dot, scratch);
-    const Z a2 = zscale(zmul(t, dot), -0.5);
-    // ---- 3. w = tau p + a2 v (registers); next column for all rows; rank-2
-    // update of the own rows; |col|^2 of the next reflector's tail
-    const Z w0c = zconj(zadd(zmul(t, p0), a2));  // v[0] = 1
-    double part = 0.;
-#pragma unroll
-    for (int q = 0; q < kPerThread; ++q) {
+    for (int q = 0; q < KP; ++q) {
       const int j = tid + q * kThreads;
       if (j < m) {
-        const Z vj = v[j];
-        const Z wj = zadd(zmul(t, pw[q]), zmul(a2, vj));
-        const Z c = zsub(pcv[q], zadd(zmul(vj, w0c), wj));
-        col[k + 1 + j] = c;
-        if (j >= 2) part += c.x * c.x + c.y * c.y;
-        pw[q] = zconj(wj);   // conj(w_j)
-        pcv[q] = zconj(vj);  // conj(v_j)
+        ok = receive(slot(k, k + 1 + j), abort_flag, p[q], c[q]) && ok;
+        p[q] = zmul(t, p[q]);  // tau p
+        dot = zadd(dot, zmul(zconj(p[q]), vj[q]));
+      }
+    }
+    dot.x = wave_sum(dot.x);
+    dot.y = wave_sum(dot.y);
+    if (lane == 0) lds.dot[wave] = dot;
+    if (!ok) expired = 1;
+    if (tid == 0) first_p = p[0];
+    __syncthreads();
+    if (expired) return;
+    // every workgroup that reads has published step k, so none reads step k - 1
+    if (tid < rpw && k > 0) {
+      const int i = g + tid * G;
+      if (i < n && i >= k) {
+        unsigned long long* s = slot(k + 2, i);
+#pragma unroll
+        for (int w = 0; w < kWords; ++w)
+          __hip_atomic_store(s + w, kMissing, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    dot = {0., 0.};
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) dot = zadd(dot, lds.dot[w]);
+    // ---- 2. w = tau p + a2 v; next column for all rows; rank-2 update of the own rows
+    const Z a2 = zscale(zmul(t, dot), -0.5);
+    const Z w0c = zconj(zadd(first_p, a2));  // v[0] = 1
+    Z wc[KP], vc[KP];
+#pragma unroll
+    for (int q = 0; q < KP; ++q) {
+      const int j = tid + q * kThreads;
+      if (j < m) {
+        const Z w = zadd(p[q], zmul(a2, vj[q]));
+        cv[q] = zsub(c[q], zadd(zmul(vj[q], w0c), w));
+        wc[q] = zconj(w);
+        vc[q] = zconj(vj[q]);
       }
     }
     for (int r = first; r < rpw; ++r) {
       const int i = g + r * G;
       if (i >= n) break;
-      const Z vi = v[i - k - 1];
-      const Z wi = zadd(zmul(t, stage_p[r - first]), zmul(a2, vi));
-      Z* row = rows + size_t(r) * n + (k + 1);
+      const Z vi = lds.v[i - k - 1];
+      const Z wi = zadd(zmul(t, lds.staged[r]), zmul(a2, vi));
+      Z* row = lds.rows + size_t(r) * n + (k + 1);
 #pragma unroll
-      for (int q = 0; q < kPerThread; ++q) {
+      for (int q = 0; q < KP; ++q) {
         const int j = tid + q * kThreads;
-        if (j < m) row[j] = zsub(row[j], zadd(zmul(vi, pw[q]), zmul(wi, pcv[q])));
+        if (j < m) row[j] = zsub(row[j], zadd(zmul(vi, wc[q]), zmul(wi, vc[q])));
       }
     }
-    const double xn2 = block_sum(part, scratch);  // also publishes col and the rows to the block
-    if (k + 2 < n) {
-      // ---- 4. next reflector and the products of step k + 1
-      t = form_reflector(col, k + 1, n, xn2, vn, refl, ldr, d, e, tau);
-      stage_products(rows, n, rpw, k + 1, vn, stage_p, stage_c, stage_i, &staged);
-    } else if (g == 0 && tid == 0) {
-      d[n - 1] = col[n - 1].x;
+    if (k + 2 == n) {
+      if (g == out && tid == 0) d[n - 1] = cv[0].x;
+      return;
     }
+    column(cv, m);
+    __builtin_amdgcn_s_waitcnt(kWaitStores);  // the refill, before the next publication
+    __syncthreads();
+    // ---- 3. next reflector and the products of step k + 1
+    t = reflect(k + 1, vj);
   }
 }
 
@@ -326,23 +311,20 @@ int device_cus() {
   return cus;
 }
 
-size_t lds_bytes(int n, int rpw) {
-  return (size_t(rpw) * n + 3 * size_t(n) + 2 * size_t(rpw)) * sizeof(Z) + 2 * kWaves * sizeof(double) +
-         size_t(rpw) * sizeof(int);
-}
-
-
-// Target rows per workgroup: 4 (measured at n = 320 / 640 / 960 against 6, 10,
-// 16 and as many as the LDS holds: 5.2 / 5.8 / 6.4 us per column, the largest
-// slabs 8.0 / 6.7 / 6.4); SDFT_HIP_HETRD_ROWS overrides. More rows are used
-// when the workgroups would outnumber the CUs.
-int target_rows_per_group() {
+// Target rows per workgroup: about 72 workgroups. More of them shorten a
+// workgroup's own work but add pollers of every published row. Measured, us per
+// column at n = 100 / 160 / 240 / 320 / 380 / 480 / 640: this rule 3.0 / 3.3 / 3.7 /
+// 4.1 / 4.2 / 4.7 / 5.0, four rows 3.1 / 3.3 / 3.7 / 4.2 / 4.5 / 4.9 / 5.8, ten rows
+// 3.6 / 3.9 / 4.2 / 4.5 / 4.6 / 4.9 / 5.1 (with arrival flags beside the values, two
+// more round trips and nine workgroup barriers a column, four rows took 4.8 / 4.9 / 5.0
+// / 5.1 / 5.2 / 5.4 / 5.7); SDFT_HIP_HETRD_ROWS overrides. More rows are used when the
+// workgroups would outnumber the CUs.
+int target_rows_per_group(int n) {
   static const int rows = [] {
     const char* e = std::getenv("SDFT_HIP_HETRD_ROWS");
-    const int v = e ? std::atoi(e) : 0;
-    return v > 0 ? v : 4;
+    return e ? std::atoi(e) : 0;
   }();
-  return rows;
+  return rows > 0 ? std::min(rows, kThreads) : std::max(1, (n + 71) / 72);
 }
 
 // LDS the kernel declares statically (the workgroup reductions of the
@@ -350,7 +332,7 @@ int target_rows_per_group() {
 size_t static_lds() {
   static const size_t bytes = [] {
     hipFuncAttributes attr{};
-    if (hipFuncGetAttributes(&attr, reinterpret_cast<const void*>(k_hetrd_lds)) != hipSuccess) return size_t(4096);
+    if (hipFuncGetAttributes(&attr, reinterpret_cast<const void*>(k_hetrd_lds<4>)) != hipSuccess) return size_t(4096);
     return size_t(attr.sharedSizeBytes);
   }();
   return bytes;
@@ -363,16 +345,17 @@ bool hetrd_plan(int n, int* rows_per_group, int* groups) {
   const size_t total = size_t(max_lds()), fixed = static_lds();
   if (fixed >= total) return false;
   const size_t budget = total - fixed;
-  // the target rows per workgroup, or more so that there is at most one
-  // workgroup per CU
-  int rpw = std::min(n, target_rows_per_group());
-  if (cus > 0) rpw = std::max(rpw, (n + cus - 1) / cus);
+  // the target rows per workgroup, as far as its LDS holds them, and at least so
+  // many that there is at most one workgroup per CU
+  const int least = cus > 0 ? (n + cus - 1) / cus : 1;
+  int rpw = std::max(std::min(n, target_rows_per_group(n)), least);
+  while (rpw > least && lds_bytes(n, rpw) > budget) --rpw;
   if (lds_bytes(n, rpw) > budget) return false;
   const int g = (n + rpw - 1) / rpw;
   if (cus > 0 && g > cus) return false;
-  // every workgroup must be resident at once (the grid barrier waits for all)
+  // every workgroup must be resident at once (each waits for all)
   int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(k_hetrd_lds), kThreads,
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(k_hetrd_lds<4>), kThreads,
                                                    lds_bytes(n, rpw)) != hipSuccess ||
       per_cu < 1 || (cus > 0 && long(per_cu) * cus < g))
     return false;
@@ -381,11 +364,9 @@ bool hetrd_plan(int n, int* rows_per_group, int* groups) {
   return true;
 }
 
-// published vectors (4 n complex), then the abort flag line, then one flag line
-// per workgroup (at most kHetrdMaxOrder workgroups)
-size_t hetrd_workspace_bytes(int n) {
-  return 4 * size_t(n) * sizeof(Z) + size_t(kFlagStride) * sizeof(unsigned) * (1 + size_t(kHetrdMaxOrder));
-}
+// the abort flag's line, then the published rows
+constexpr size_t kFlagBytes = 64;
+size_t hetrd_workspace_bytes(int n) { return kFlagBytes + kBuffers * kWords * size_t(n) * sizeof(unsigned long long); }
 
 hipError_t launch_hetrd(const double* a, long lda, int n, double* refl, long ldr, double* d, double* e, double* tau,
                         void* workspace, hipStream_t s, bool force_expiry) {
@@ -395,14 +376,13 @@ hipError_t launch_hetrd(const double* a, long lda, int n, double* refl, long ldr
     // d = Re a; nothing to reduce
     return hipMemcpyAsync(d, a, sizeof(double), hipMemcpyDeviceToDevice, s);
   }
-  Z* pub_p = reinterpret_cast<Z*>(workspace);
-  Z* pub_c = pub_p + 2 * size_t(n);
-  int* abort_flag = reinterpret_cast<int*>(pub_c + 2 * size_t(n));
-  unsigned* flags = reinterpret_cast<unsigned*>(abort_flag) + kFlagStride;
-  hipError_t err = hipMemsetAsync(abort_flag, 0, size_t(kFlagStride) * sizeof(unsigned) * (1 + size_t(groups)), s);
+  int* abort_flag = reinterpret_cast<int*>(workspace);
+  auto* pub = reinterpret_cast<unsigned long long*>(static_cast<char*>(workspace) + kFlagBytes);
+  // one fill: nothing published, nobody gave up (kHetrdRunning)
+  hipError_t err = hipMemsetAsync(workspace, 0xFF, hetrd_workspace_bytes(n), s);
   if (err != hipSuccess) return err;
   // host-forced expiry (fault injection): the abort flag is raised before the
-  // launch, so every workgroup leaves at its first wait and the kernel ends
+  // launch, so workgroups leave at their waits and the result is discarded
   if (force_expiry && (err = hipMemsetAsync(abort_flag, 1, 1, s)) != hipSuccess) return err;
   const Z* az = reinterpret_cast<const Z*>(a);
   Z* rz = reinterpret_cast<Z*>(refl);
@@ -413,21 +393,22 @@ hipError_t launch_hetrd(const double* a, long lda, int n, double* refl, long ldr
   // redoes the solve by divide and conquer. A cooperative launch would
   // instead serialise the device for the reduction, and it is refused when
   // several processes share the device.
-  hipLaunchKernelGGL(k_hetrd_lds, dim3(groups), dim3(kThreads), lds_bytes(n, rpw), s, az, lda, n, rpw, rz, ldr, d, e,
-                     tz, pub_p, pub_c, flags, abort_flag);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(groups), dim3(kThreads), lds_bytes(n, rpw), s, az, lda, n, rpw, rz, ldr, d, e, tz, pub,
+                       abort_flag);
+  };
+  if (n <= kThreads) go(k_hetrd_lds<1>);
+  else if (n <= 2 * kThreads) go(k_hetrd_lds<2>);
+  else go(k_hetrd_lds<4>);
   return hipGetLastError();
 }
 
-const int* hetrd_abort_flag(const void* workspace, int n) {
-  const Z* pub = reinterpret_cast<const Z*>(workspace);
-  return reinterpret_cast<const int*>(pub + 4 * size_t(n));
-}
-
+const int* hetrd_abort_flag(const void* workspace, int) { return reinterpret_cast<const int*>(workspace); }
 
 // Loads this file's code object on the calling thread (see module_prime.hpp).
 hipError_t prime_module_tridiag() {
   hipFuncAttributes a{};
-  return hipFuncGetAttributes(&a, reinterpret_cast<const void*>(k_hetrd_lds));
+  return hipFuncGetAttributes(&a, reinterpret_cast<const void*>(k_hetrd_lds<4>));
 }
 
 }  // namespace sdft_hip

@@ -91,16 +91,16 @@ std::vector<double> HermitianEigensolver::solve(const double* a, long m, long k,
   return std::vector<double>(h.begin() + 8, h.begin() + 8 + count);
 }
 
-// Synchronises the stream; true when the reduction's bounded grid barrier
+// Synchronises the stream; true when one of the reduction's bounded waits
 // expired (its outputs are then invalid).
 bool HermitianEigensolver::barrier_expired(long m) {
-  int aborted = 0;
+  int flag = kHetrdRunning;
   if (m > 1)
-    check(hipMemcpyAsync(&aborted, hetrd_abort_flag(work_.p, int(m)), sizeof(int), hipMemcpyDeviceToHost,
+    check(hipMemcpyAsync(&flag, hetrd_abort_flag(work_.p, int(m)), sizeof(int), hipMemcpyDeviceToHost,
                          ctx_.stream()),
           "abort flag");
   ctx_.sync();
-  return aborted != 0;
+  return flag != kHetrdRunning;
 }
 
 // rocSOLVER zheevd on a copy of `a` (orders above the one-launch reduction's

@@ -368,6 +368,8 @@ __global__ void k_atom_blocks_f32(int np, int columns, int atoms, const int* __r
   }
 }
 
+unsigned reduce_blocks(int M, int N) { return unsigned(std::min<long>(1024, (long(M) * N + 255) / 256)); }
+
 // Tiles: 0 = 32 x 32, 1 = 64 x 32, 2 = 64 x 64.
 struct Tile {
   int bm, bn;
@@ -425,11 +427,15 @@ long tile_count(int M, int N, int cfg) {
 }
 // Splits along K for about 1200 workgroups (a little over four a CU; 512 x 160 x n took
 // 213 us with 1280, 230 and more with 640), at least 256 of K each, or 128 while that
-// leaves CUs without a workgroup (128 x 37 x 4573 in 32 splits of 143); 48 at most.
+// leaves CUs without a workgroup (128 x 37 x 4573 in 32 splits of 143), or 64 while half
+// of them have none: a slab of K is then a round trip to memory, and the reduction of
+// more partials costs less (120 x 20 x 1647 in 12 / 26 splits 12.6 / 9.7 us, 20 x 20 x 1647
+// 13.6 / 9.2, 64 x 4 x 1647 11.8 / 8.8, 160 x 160 x 160 in 1 / 2 10.2 / 8.6); 48 at most.
 int splits_for(long tiles, int K) {
   const long most = std::min<long>(48, (1200 + tiles - 1) / tiles);
-  long splits = std::min<long>(most, std::max<long>(1, K / 256));
-  if (tiles * splits < 256) splits = std::min<long>(most, std::max<long>(1, K / 128));
+  long splits = std::min<long>(most, K / 256);
+  if (tiles * splits < 256) splits = std::min<long>(most, K / 128);
+  if (tiles * splits < 128) splits = std::min<long>({most, K / 64, (256 + tiles - 1) / tiles});
   return int(std::max<long>(1, splits));
 }
 // The tile of a shape, for both precisions: 64 x 64 where the result is wide (256
@@ -488,7 +494,8 @@ hipError_t run(int aop, int bop, int M, int N, int K, double alpha, const TA* A,
                                                    n_first, alpha, pl.kps, wk, s, ev);
   if (partials) *partials = pl.splits;
   if (e != hipSuccess || pl.splits == 1 || partials) return e;
-  hipLaunchKernelGGL(k_splitk_reduce, dim3(1024), dim3(256), 0, s, M, N, pl.splits, work, first, second, n_first);
+  hipLaunchKernelGGL(k_splitk_reduce, dim3(reduce_blocks(M, N)), dim3(256), 0, s, M, N, pl.splits, work, first, second,
+                     n_first);
   return hipGetLastError();
 }
 }  // namespace
@@ -724,7 +731,7 @@ hipError_t zgemm_bf16_storage(int aop, int M, int N, int K, double alpha, const 
   if (partials) *partials = splits;
   if (e != hipSuccess || splits == 1 || partials) return e;
   const GemmOutput o{C, ldc, D, ldd, beta};
-  hipLaunchKernelGGL(k_splitk_reduce, dim3(1024), dim3(256), 0, s, M, N, splits, work, o, o, N);
+  hipLaunchKernelGGL(k_splitk_reduce, dim3(reduce_blocks(M, N)), dim3(256), 0, s, M, N, splits, work, o, o, N);
   return hipGetLastError();
 }
 

@@ -299,7 +299,8 @@ int sdft_hip_local_hamiltonian(sdft_hip_context* ctx, const int shape[3], const 
       cx.record("gpu_fft_operator_upload_saved", 0, count + npw);
     }
     L.kinetic.upload(kinetic, npw, s);  // kinetic stays dynamic (src/compute_backend.hpp:43-44)
-    L.in.upload(input, 2 * npw * columns, s);
+    L.in.reserve(2 * npw * columns);
+    cx.upload_bulk(L.in.p, input, 16 * npw * columns);
     L.out.reserve(2 * npw * columns);
     const std::size_t per_col = std::size_t(L.grid.dev.nsticks) * shp[2] * 16;
     const std::size_t chunk = std::max<std::size_t>(1, std::min<std::size_t>(columns, (std::size_t(512) << 20) / per_col));
@@ -316,8 +317,7 @@ int sdft_hip_local_hamiltonian(sdft_hip_context* ctx, const int shape[3], const 
         check(sdft_hip::launch_local_h<float>(L.grid.dev, x, long(npw), c, L.kinetic.p, y, long(npw), L.t1.p, L.t2.p, s),
               "local H");
     }
-    check(hipMemcpyAsync(output, L.out.p, 16 * npw * columns, hipMemcpyDeviceToHost, s), "copy out");
-    cx.sync();
+    cx.download_bulk(output, L.out.p, 16 * npw * columns);
     L.identity = operator_identity;
     cx.record(prec == Precision::FP64 ? "hip_fp64_fft_dispatch" : "hip_fp32_fft_dispatch", 0);
   });
@@ -355,7 +355,8 @@ int sdft_hip_paw_pair(sdft_hip_context* ctx, uint64_t identity, size_t npw, size
     } else {
       cx.record("gpu_paw_chain_density_hit", 0);
     }
-    P.in.upload(input, 2 * npw * columns, st);
+    P.in.reserve(2 * npw * columns);
+    cx.upload_bulk(P.in.p, input, 16 * npw * columns);
     P.p.reserve(2 * np * columns);
     P.dq.reserve(4 * np * columns);
     P.h.reserve(2 * npw * columns);
@@ -368,9 +369,8 @@ int sdft_hip_paw_pair(sdft_hip_context* ctx, uint64_t identity, size_t npw, size
     double* hs = P.h.p;
     cx.zgemm(prec, 1, 0, K, N, M, 1.0, P.b.p, M, P.dq.p, M, hs, K, nullptr, 0, 0.0);
     cx.zgemm(prec, 1, 0, K, N, M, 1.0, P.b.p, M, P.dq.p + 2 * M * N, M, P.s.p, K, nullptr, 0, 0.0);
-    check(hipMemcpyAsync(h, P.h.p, 16 * npw * columns, hipMemcpyDeviceToHost, st), "copy h");
-    check(hipMemcpyAsync(s_out, P.s.p, 16 * npw * columns, hipMemcpyDeviceToHost, st), "copy s");
-    cx.sync();
+    cx.download_bulk(h, P.h.p, 16 * npw * columns);
+    cx.download_bulk(s_out, P.s.p, 16 * npw * columns);
     P.identity = identity;
     P.projector_identity = projector_identity;
     P.npw = npw;

@@ -111,8 +111,9 @@ class Context {
   // pinned staging of the main stream's control transfers (allocated once)
   PinnedStaging& staging();
   // bulk transfers between pageable host memory and the device on the main
-  // stream through two pinned chunks: the DMA of one chunk overlaps the host
-  // copy of the other. Both return with the transfer complete.
+  // stream through pinned chunks: the DMA of one chunk overlaps the host copy
+  // of another. An upload returns once host_src is free to change (the device
+  // has it in the stream's order), a download with the transfer complete.
   void upload_bulk(void* device_dst, const void* host_src, std::size_t bytes);
   void download_bulk(void* host_dst, const void* device_src, std::size_t bytes);
   rocblas_handle blas() const { return blas_; }
@@ -185,9 +186,13 @@ class Context {
   int device_;
   hipStream_t stream_{};
   std::unique_ptr<PinnedStaging> staging_;
-  char* bulk_[2] = {nullptr, nullptr};
-  hipEvent_t bulk_done_[2] = {};
+  static constexpr int kBulkBuffers = 4;
+  char* bulk_ = nullptr;
+  hipEvent_t bulk_done_[kBulkBuffers] = {};
+  bool bulk_busy_[kBulkBuffers] = {};  // a DMA of the chunk may be under way
+  int bulk_next_ = 0;
   void bulk_buffers();
+  int bulk_issue(void* dst, const void* src, std::size_t len, bool to_device);
   rocblas_handle blas_{};
   std::string name_;
   char* scratch_ = nullptr;

@@ -343,7 +343,7 @@ class Context:
         kin = np.ascontiguousarray(kinetic, dtype=np.float64)
         pot = np.ascontiguousarray(potential, dtype=np.float64)
         x = np.asfortranarray(x, dtype=np.complex128)
-        out = np.zeros_like(x, order="F")
+        out = np.empty_like(x, order="F")
         _check(lib().sdft_hip_local_hamiltonian(self.handle, _p(shp, _ip), _p(idx, _u64p), ct.c_size_t(len(idx)),
                                                 _p(kin), _p(pot), _p(x), ct.c_size_t(x.shape[1]), _p(out),
                                                 ct.c_uint64(operator_identity), ct.c_int(precision)))
@@ -355,8 +355,8 @@ class Context:
         q = np.asfortranarray(q, dtype=np.complex128)
         x = np.asfortranarray(x, dtype=np.complex128)
         npj, npw = b.shape
-        h = np.zeros((npw, x.shape[1]), dtype=np.complex128, order="F")
-        s = np.zeros_like(h)
+        h = np.empty((npw, x.shape[1]), dtype=np.complex128, order="F")
+        s = np.empty_like(h)
         handled = ct.c_int()
         _check(lib().sdft_hip_paw_pair(self.handle, ct.c_uint64(identity), ct.c_size_t(npw), ct.c_size_t(npj),
                                        ct.c_size_t(x.shape[1]), _p(b), _p(d), _p(q), _p(x), _p(h), _p(s),
@@ -692,8 +692,8 @@ class Batch:
         x = np.zeros(int(self.offsets[-1]), dtype=np.complex128)
         for k, b in enumerate(blocks):
             x[self.offsets[k]:self.offsets[k + 1]] = np.asfortranarray(b, dtype=np.complex128).ravel(order="F")
-        hy = np.zeros_like(x)
-        sy = np.zeros_like(x)
+        hy = np.empty_like(x)
+        sy = np.empty_like(x)
         _check(lib().sdft_hip_batch_apply(self.handle, _p(x), _p(hy), _p(sy)))
         split = lambda a: [a[self.offsets[k]:self.offsets[k + 1]].reshape(self.columns, -1).T
                            for k in range(len(self.operators))]

@@ -29,30 +29,30 @@ def local(si8):
     return synthetic.dense_operator(bare)[0]
 
 
-@pytest.mark.parametrize("rows", sorted(ROWS))
-@pytest.mark.parametrize("columns", [1, 21])
-@pytest.mark.parametrize("precision", [0, 1])
-def test_onsite_groups(hip_ctx, si8, local, rows, columns, precision, monkeypatch):
+# chunk 4: H in passes of 4 columns at most, S in one
+@pytest.mark.parametrize("rows,chunk", [(r, None) for r in sorted(ROWS)] + [("groups", "4")])
+def test_onsite_groups(hip_ctx, si8, local, rows, chunk, monkeypatch):
     from sdft_amd import native
+    if chunk:
+        monkeypatch.setenv("SDFT_HIP_APPLY_CHUNK", chunk)
     prob = _problem(si8, ROWS[rows])
-    rng = np.random.default_rng(columns)
-    x = rng.standard_normal((prob.n, columns)) + 1j * rng.standard_normal((prob.n, columns))
-    theta = rng.standard_normal(columns)
-    b = prob.all_b()
-    onsite = lambda blocks: b.conj().T @ (blocks @ (b @ x))
-    want = dict(h=local @ x + onsite(prob.block_d()), s=(1 + prob.regularization) * x + onsite(prob.block_q()))
-    want["shifted"] = want["h"] - want["s"] * theta
-    # chains of n terms in the projection and of the atom's rows twice over, by steps
-    # that grow like a random walk
-    tol = 8 * (2.0 ** -53 if precision == 0 else 2.0 ** -24) * prob.n ** 0.5
-    near = lambda got, key: np.linalg.norm(got - want[key]) <= tol * np.linalg.norm(want[key])
-    for chunk in (None, "4"):  # "4": H in passes of 4 columns at most, S in one
-        if chunk:
-            monkeypatch.setenv("SDFT_HIP_APPLY_CHUNK", chunk)
-        op = native.Operator(hip_ctx, prob)
-        hy, sy = op.apply(x, precision=precision)
-        assert near(hy, "h") and near(sy, "s")
-        assert near(op.apply(x, which="h", precision=precision), "h")
-        assert near(op.apply(x, which="s", precision=precision), "s")
-        assert near(op.apply_shifted(x, theta, precision=precision), "shifted")
-        op.close()
+    b, d, q = prob.all_b(), prob.block_d(), prob.block_q()
+    op = native.Operator(hip_ctx, prob)
+    for columns in (1, 21):
+        rng = np.random.default_rng(columns)
+        x = rng.standard_normal((prob.n, columns)) + 1j * rng.standard_normal((prob.n, columns))
+        theta = rng.standard_normal(columns)
+        want = dict(h=local @ x + b.conj().T @ (d @ (b @ x)),
+                    s=(1 + prob.regularization) * x + b.conj().T @ (q @ (b @ x)))
+        want["shifted"] = want["h"] - want["s"] * theta
+        for precision in (0, 1):
+            # chains of n terms in the projection and of the atom's rows twice over, by steps
+            # that grow like a random walk
+            tol = 8 * (2.0 ** -53 if precision == 0 else 2.0 ** -24) * prob.n ** 0.5
+            near = lambda got, key: np.linalg.norm(got - want[key]) <= tol * np.linalg.norm(want[key])
+            hy, sy = op.apply(x, precision=precision)
+            assert near(hy, "h") and near(sy, "s"), (columns, precision)
+            assert near(op.apply(x, which="h", precision=precision), "h"), (columns, precision)
+            assert near(op.apply(x, which="s", precision=precision), "s"), (columns, precision)
+            assert near(op.apply_shifted(x, theta, precision=precision), "shifted"), (columns, precision)
+    op.close()

@@ -234,9 +234,9 @@ __device__ __forceinline__ void y_out(cx<T>* rows, const PlaneRows& pr, const Bu
 // 160 columns of 72^3 627 -> 304 us FP64 and 301 -> 162 us FP32, 96 columns of
 // 48 x 48 x 96 311 -> 222 us FP64, 37 columns of 70 x 35 x 35 56 -> 42 us FP64;
 // without the dropped digits, the branch-free gathers and the loads ahead of the
-// barriers 371, 186, 238 and 44. The FP64 kernel without the empty middle is kept to the
-// registers of three waves a SIMD (168): 222 -> 198 us on the slab, 42 -> 38 on 70 x 35,
-// unchanged on 72 x 72, where LDS allows two.
+// barriers 371, 186, 238 and 44. HALF, which drops the empty middle, is kept to the registers
+// of three waves a SIMD (168; the full kernel would spill): FP64 222 -> 198 us on the slab,
+// 42 -> 38 on 70 x 35, unchanged on 72 x 72, where LDS allows two.
 template <typename T, bool WIDE, bool HALF>
 __global__ __launch_bounds__(WIDE ? 256 : 512) __attribute__((amdgpu_waves_per_eu(WIDE ? 1 : HALF ? 3 : 2))) void k_plane_local(
     const cx<T>* __restrict__ t1, cx<T>* __restrict__ t2, const int* __restrict__ stick_map, int nsticks, int n0,

@@ -21,9 +21,9 @@
 // they have arrived. A word not yet published is all ones (a NaN that is never
 // published); three buffers take turns, and a workgroup refills its own
 // entries of the one that every other has left, completed before its next
-// publication. A workgroup without rows left leaves the kernel, so that whoever
-// still reads a step has published the step before. Waits are bounded: on expiry an
-// abort flag ends every workgroup.
+// publication. A workgroup leaves before a step that it would read without publishing
+// the next (tridiag_exchange.hpp), so that whoever has all of step k knows that nobody
+// reads step k - 1. Waits are bounded: on expiry an abort flag ends every workgroup.
 // Every published word is stored and loaded with agent-scope relaxed atomics
 // (sc1 accesses, coherent across the XCDs' L2 caches), which needs no L2 write-back
 // or invalidate (an agent-scope fence would issue one on every column).
@@ -33,6 +33,7 @@
 #include <cstdlib>
 
 #include "tridiag.hpp"
+#include "tridiag_exchange.hpp"
 #include "wave_sum.hpp"
 
 namespace sdft_hip {
@@ -42,7 +43,6 @@ constexpr int kThreads = 512;
 constexpr int kWaves = kThreads / 64;
 constexpr long kSpinLimit = 1L << 20;
 constexpr unsigned long long kMissing = ~0ull;  // a published word that has not arrived
-constexpr int kBuffers = 3;
 constexpr int kWords = 4;  // of one published row: p_i, A_{i,k+1}
 
 // Aligned to 16 bytes: one element is one 128-bit LDS access (the dynamic LDS
@@ -123,9 +123,9 @@ __global__ __launch_bounds__(kThreads) void k_hetrd_lds(const Z* __restrict__ a,
   __shared__ Z first_p;  // tau p of the first row
   const HetrdLds lds(lds_raw, n, rpw);
   const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int out = (n - 1) % G;  // the workgroup of the last row writes d, e, tau and the reflectors
-  auto slot = [&](int step, int row) { return pub + kWords * (size_t(step % kBuffers) * n + row); };
-  auto first_row = [&](int i0) { return i0 <= g ? 0 : (i0 - g + G - 1) / G; };  // first r with g + r G >= i0
+  const int out = hetrd_last_group(n, G);  // writes d, e, tau and the reflectors
+  auto slot = [&](int step, int row) { return pub + kWords * (size_t(step % kHetrdBuffers) * n + row); };
+  auto first_row = [&](int i0) { return hetrd_first_row(G, g, i0); };  // first r with g + r G >= i0
 
   // Reflector of the column in lds.col at rows c0 + 1 .. n - 1 (LAPACK zlarfg
   // conventions; |tail|^2 as wave partials in lds.norm, the workgroup's barrier
@@ -219,7 +219,7 @@ __global__ __launch_bounds__(kThreads) void k_hetrd_lds(const Z* __restrict__ a,
   Z t = reflect(0, vj);
   for (int k = 0; k + 1 < n; ++k) {
     const int m = n - k - 1, first = first_row(k + 1);
-    if (first >= rpw || g + first * G >= n) return;  // no row left (the last row's workgroup stays)
+    if (!hetrd_reads(n, G, g, k)) return;
     // ---- 1. the published products of every row; partial (tau p)^H v
     Z p[KP], c[KP];
     bool ok = true;
@@ -240,7 +240,7 @@ __global__ __launch_bounds__(kThreads) void k_hetrd_lds(const Z* __restrict__ a,
     if (tid == 0) first_p = p[0];
     __syncthreads();
     if (expired) return;
-    // every workgroup that reads has published step k, so none reads step k - 1
+    // step k is complete, so nobody reads step k - 1 (hetrd_reads): its buffer is free
     if (tid < rpw && k > 0) {
       const int i = g + tid * G;
       if (i < n && i >= k) {
@@ -366,7 +366,7 @@ bool hetrd_plan(int n, int* rows_per_group, int* groups) {
 
 // the abort flag's line, then the published rows
 constexpr size_t kFlagBytes = 64;
-size_t hetrd_workspace_bytes(int n) { return kFlagBytes + kBuffers * kWords * size_t(n) * sizeof(unsigned long long); }
+size_t hetrd_workspace_bytes(int n) { return kFlagBytes + kHetrdBuffers * kWords * size_t(n) * sizeof(unsigned long long); }
 
 hipError_t launch_hetrd(const double* a, long lda, int n, double* refl, long ldr, double* d, double* e, double* tau,
                         void* workspace, hipStream_t s, bool force_expiry) {

@@ -82,12 +82,14 @@ __device__ __forceinline__ void backward(cx<T>* lines, const double* __restrict_
   }
 }
 
-// a / b with inv = 1 / b rounded: the quotient corrected once by its exact
-// residual is the rounded quotient (Markstein, IBM J. Res. Dev. 34, 1990), in three
-// operations instead of the compiler's general division.
+// a / b with inv = 1 / b rounded, for a count b: the quotient corrected once by its
+// exact residual is the rounded quotient (Markstein, IBM J. Res. Dev. 34, 1990), in
+// three operations and a select instead of the compiler's general division. An
+// infinite a has no residual (inf - inf): its quotient stands.
 __device__ __forceinline__ double divide(double a, double b, double inv) {
   const double q = a * inv;
-  return __builtin_fma(__builtin_fma(-q, b, a), inv, q);
+  const double rounded = __builtin_fma(__builtin_fma(-q, b, a), inv, q);
+  return __builtin_isinf(q) ? q : rounded;
 }
 
 // t2[column][z slot][stick], slot -> natural order, onto the sphere:

@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include "gemm.hpp"
+#include "gemm_plan.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -19,7 +20,7 @@
 namespace sdft_hip {
 
 namespace {
-constexpr int BK = 16;  // K of one slab
+constexpr int BK = kGemmSlab;  // K of one slab
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
@@ -370,12 +371,6 @@ __global__ void k_atom_blocks_f32(int np, int columns, int atoms, const int* __r
 
 unsigned reduce_blocks(int M, int N) { return unsigned(std::min<long>(1024, (long(M) * N + 255) / 256)); }
 
-// Tiles: 0 = 32 x 32, 1 = 64 x 32, 2 = 64 x 64.
-struct Tile {
-  int bm, bn;
-};
-constexpr Tile kTiles[3] = {{32, 32}, {64, 32}, {64, 64}};
-
 template <typename T, typename TA, typename TB, int CFG, bool FAR>
 hipError_t launch_cfg(int aop, int bop, dim3 grid, int M, int N, int K, const TA* A, long lda, const TB* B, long ldb,
                       const GemmOutput& first, const GemmOutput& second, int n_first, double alpha, int kps,
@@ -417,55 +412,15 @@ hipError_t dispatch_ops(int cfg, int aop, int bop, dim3 grid, int M, int N, int 
   return hipEventRecord(ev->end, s);
 }
 
-// Split-K plan of a shape: tile configuration, splits and K per split.
-struct Plan {
+// The launch of a plan; without a workspace the product is not split.
+struct Launch {
   int cfg, splits, kps;
   dim3 grid;
 };
-long tile_count(int M, int N, int cfg) {
-  return long((M + kTiles[cfg].bm - 1) / kTiles[cfg].bm) * ((N + kTiles[cfg].bn - 1) / kTiles[cfg].bn);
-}
-// Splits along K for about 1200 workgroups (a little over four a CU; 512 x 160 x n took
-// 213 us with 1280, 230 and more with 640), at least 256 of K each, or 128 while that
-// leaves CUs without a workgroup (128 x 37 x 4573 in 32 splits of 143), or 64 while half
-// of them have none: a slab of K is then a round trip to memory, and the reduction of
-// more partials costs less (120 x 20 x 1647 in 12 / 26 splits 12.6 / 9.7 us, 20 x 20 x 1647
-// 13.6 / 9.2, 64 x 4 x 1647 11.8 / 8.8, 160 x 160 x 160 in 1 / 2 10.2 / 8.6); 48 at most.
-int splits_for(long tiles, int K) {
-  const long most = std::min<long>(48, (1200 + tiles - 1) / tiles);
-  long splits = std::min<long>(most, K / 256);
-  if (tiles * splits < 256) splits = std::min<long>(most, K / 128);
-  if (tiles * splits < 128) splits = std::min<long>({most, K / 64, (256 + tiles - 1) / tiles});
-  return int(std::max<long>(1, splits));
-}
-// The tile of a shape, for both precisions: 64 x 64 where the result is wide (256
-// columns, at most a tenth of them padding) and has 1200 such tiles, 64 x 32 where
-// 768 workgroups are reached with splits, else 32 x 32. Measured, us, 64 x 64 /
-// 64 x 32 / 32 x 32 at their best splits (n = 23847): n x 480 x 512 adjoint FP64
-// 687 / 749 / 777, FP32 373 / 433 / 494; 512 x 160 x n FP64 268 / 213 / 225, FP32
-// 140 / 126 / 133; 640 x 160 x n FP64 331 / 299 / 299, FP32 183 / 176 / 197; n x 220 x
-// 380 FP64 279 / 260 / 267; 160 x 160 x n FP64 116 / 95 / 85; 128 x 37 x 4573 FP64
-// 25 / 17 / 13; 9141 x 80 x 256 adjoint FP64 57 / 38 / 37. Against the single-buffered
-// kernels (32 x 32 and 128 x 32 tiles, two barriers and per-element addresses and
-// bounds in every slab): 512 x 160 x n FP64 287, FP32 164; 640 x 160 x n 391, 236;
-// n x 480 x 512 823, 562; 160 x 160 x n 101, 69; 128 x 37 x 4573 19, 16.
-Plan plan_shape(int M, int N, int K) {
-  Plan p{};
-  p.cfg = 0;
-  if (N >= 256 && (N + 63) / 64 * 64 <= N + N / 10 && tile_count(M, N, 2) >= 1200) {
-    p.cfg = 2;
-  } else {
-    const long tiles = tile_count(M, N, 1);
-    if (tiles * splits_for(tiles, K) >= 768) p.cfg = 1;
-  }
-  p.splits = splits_for(tile_count(M, N, p.cfg), K);
-  return p;
-}
-Plan plan_for(int M, int N, int K, bool have_work) {
-  Plan p = plan_shape(M, N, K);
-  if (p.splits > 1 && !have_work) p.splits = 1;
-  p.kps = (K + p.splits - 1) / p.splits;
-  p.kps = ((p.kps + BK - 1) / BK) * BK;
+Launch launch_for(const GemmPlan& plan, int M, int N, int K, bool have_work) {
+  Launch p{};
+  p.cfg = plan.cfg;
+  p.kps = have_work ? plan.kps : gemm_k_per_split(K, 1);
   p.splits = (K + p.kps - 1) / p.kps;
   p.grid = dim3((M + kTiles[p.cfg].bm - 1) / kTiles[p.cfg].bm, (N + kTiles[p.cfg].bn - 1) / kTiles[p.cfg].bn,
                 p.splits);
@@ -480,7 +435,8 @@ std::size_t zgemm_workspace_bytes(int M, int N, int K) {
   return splits > 1 ? std::size_t(splits) * M * N * 16 : 0;
 }
 
-int zgemm_splits(int M, int N, int K) { return K > 0 ? plan_shape(M, N, K).splits : 1; }
+// FP64 splits at least as often as FP32
+int zgemm_splits(int M, int N, int K) { return K > 0 ? gemm_plan(true, M, N, K).splits : 1; }
 
 namespace {
 template <typename T, typename TA>
@@ -488,7 +444,7 @@ hipError_t run(int aop, int bop, int M, int N, int K, double alpha, const TA* A,
                const GemmOutput& first, const GemmOutput& second, int n_first, double* work, std::size_t work_bytes,
                hipStream_t s, const LaunchEvents* ev, int* partials) {
   const bool room = work != nullptr && work_bytes >= zgemm_workspace_bytes(M, N, K);
-  const Plan pl = plan_for(M, N, K, room);
+  const Launch pl = launch_for(gemm_plan(sizeof(T) == 8, M, N, K), M, N, K, room);
   double* wk = pl.splits > 1 ? work : nullptr;
   const hipError_t e = dispatch_ops<T, TA, double>(pl.cfg, aop, bop, pl.grid, M, N, K, A, lda, B, ldb, first, second,
                                                    n_first, alpha, pl.kps, wk, s, ev);

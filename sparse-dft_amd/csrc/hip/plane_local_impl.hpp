@@ -14,6 +14,7 @@
 //   y out  first step in `rows`, last step from registers straight to T2.
 #pragma once
 #include "local_h.hpp"
+#include "plane_plan.hpp"
 #include "sphere_fft.hpp"
 #include "sphere_fft_device.hpp"
 
@@ -229,14 +230,15 @@ __device__ __forceinline__ void y_out(cx<T>* rows, const PlaneRows& pr, const Bu
 }
 
 // grid (n2 z slots, columns). Bound: vector issue in FP32 (95 % of the cycles),
-// latency in FP64 (half of them; two waves a SIMD fit the registers and LDS); HBM
-// carries only the sticks. Measured alone, in-place plane kernel -> this one:
-// 160 columns of 72^3 627 -> 304 us FP64 and 301 -> 162 us FP32, 96 columns of
-// 48 x 48 x 96 311 -> 222 us FP64, 37 columns of 70 x 35 x 35 56 -> 42 us FP64;
-// without the dropped digits, the branch-free gathers and the loads ahead of the
-// barriers 371, 186, 238 and 44. HALF, which drops the empty middle, is kept to the registers
-// of three waves a SIMD (168; the full kernel would spill): FP64 222 -> 198 us on the slab,
-// 42 -> 38 on 70 x 35, unchanged on 72 x 72, where LDS allows two.
+// latency in FP64 (half of them; the registers hold three waves a SIMD, the LDS two of
+// them at 72 x 72); HBM carries only the sticks. Measured alone, in-place plane kernel ->
+// this one: 160 columns of 72^3 627 -> 308 us FP64 and 301 -> 163 us FP32, 96 columns of
+// 48 x 48 x 96 311 -> 121 us FP64, 37 columns of 70 x 35 x 35 56 -> 26 us FP64; without
+// the dropped digits, the branch-free gathers, the loads ahead of the barriers and the
+// bounds below 371, 186, 238 and 44. HALF, which drops the empty middle, is kept to the
+// registers of three waves a SIMD (168 in FP64, six more spilled: 28 bytes a lane; the
+// full kernel would spill 46): 222 -> 198 us on 48 x 48 with two of them resident, 121
+// with three, unchanged on 72 x 72.
 template <typename T, bool WIDE, bool HALF>
 __global__ __launch_bounds__(WIDE ? 256 : 512) __attribute__((amdgpu_waves_per_eu(WIDE ? 1 : HALF ? 3 : 2))) void k_plane_local(
     const cx<T>* __restrict__ t1, cx<T>* __restrict__ t2, const int* __restrict__ stick_map, int nsticks, int n0,
@@ -273,7 +275,16 @@ __global__ __launch_bounds__(WIDE ? 256 : 512) __attribute__((amdgpu_waves_per_e
 #undef SDFT_HIP_Y_OUT
 }
 
-constexpr int kLdsPerCu = 160 * 1024;
+// Waves of the kernel that a CU's registers hold (8 where the runtime does not say)
+template <typename T, bool WIDE, bool HALF>
+int register_waves() {
+  static const int waves = [] {
+    int groups = 0;
+    const void* kernel = reinterpret_cast<const void*>(k_plane_local<T, WIDE, HALF>);
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&groups, kernel, 256, 0) == hipSuccess && groups > 0 ? 4 * groups : 8;
+  }();
+  return waves;
+}
 
 }  // namespace plane_local
 
@@ -295,24 +306,14 @@ bool plan_plane_local(const GridPlanDev& p, PlaneLocalPlan& plan) {
   plan.wide = wide_split(a0, b0) || wide_split(a1, b1);
   plan.half = !plan.wide && half_empty(a0, b0, plan.low, plan.high) && half_empty(a1, b1, p.ylow, p.yhigh);
   plan.buffer_elements = p.n0 * (64 / (a0 > b0 ? a0 : b0));
-  // the wave count that puts most waves on a CU, up to the 16 that its registers
-  // hold; the smaller workgroup where both do (FP64 up to about 72 x 72: four
-  // waves, two workgroups a CU; above, one workgroup fits and eight waves share it)
-  int best = 0;
-  for (int nw : {4, 8}) {
-    if (nw == 8 && plan.wide) break;  // its registers fit four waves
-    const std::size_t lds =
-        (std::size_t(rows + 2) * line_stride(p.n1) + std::size_t(nw) * plan.buffer_elements) * sizeof(cx<T>);
-    if (lds > std::size_t(max_lds_bytes())) continue;
-    const int waves = int(std::size_t(plane_local::kLdsPerCu) / lds) * nw;
-    const int useful = waves < 16 ? waves : 16;
-    if (useful > best) {
-      best = useful;
-      plan.waves = nw;
-      plan.lds_bytes = lds;
-    }
-  }
-  return best > 0;
+  const std::size_t fixed = std::size_t(rows + 2) * line_stride(p.n1) * sizeof(cx<T>);
+  const std::size_t per_wave = std::size_t(plan.buffer_elements) * sizeof(cx<T>);
+  const int registers = plan.wide   ? plane_local::register_waves<T, true, false>()
+                        : plan.half ? plane_local::register_waves<T, false, true>()
+                                    : plane_local::register_waves<T, false, false>();
+  plan.waves = plane_group_waves(fixed, per_wave, std::size_t(max_lds_bytes()), registers, plan.wide ? 4 : 8);
+  plan.lds_bytes = fixed + std::size_t(plan.waves) * per_wave;
+  return plan.waves > 0;
 }
 
 template <typename T>

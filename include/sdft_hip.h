@@ -403,9 +403,16 @@ int sdft_hip_strict_step(sdft_hip_operator* op, int kind, size_t roots, double t
                          const double* direction, double* energies, double* residual_norms, int* accepted);
 
 /* Compensated per-atom onsite products W = [D_a P_a | Q_a P_a] on the device
- * (src/paw_compensated_product.hpp:110-135 order), host pointers; for tests. */
+ * (src/paw_compensated_product.hpp:110-135 order), host pointers, by the kernel that
+ * an application of these atoms takes; for tests. */
 int sdft_hip_onsite_blocks(sdft_hip_context* ctx, size_t atoms, const long* rows, const double* d, const double* q,
                            const double* p, size_t columns, double* w, int precision);
+/* The same with P given as `splits` partial sums, one block np x columns after the
+ * other (np: the atoms' rows together): an application's split projection; for tests.
+ * SDFT_HIP_INVALID_ARGUMENT where the application does not sum them itself (an atom
+ * of more than 1024 rows, more than 65535 columns). */
+int sdft_hip_onsite_partials(sdft_hip_context* ctx, size_t atoms, const long* rows, const double* d, const double* q,
+                             size_t splits, const double* partials, size_t columns, double* w, int precision);
 
 #ifdef __cplusplus
 }

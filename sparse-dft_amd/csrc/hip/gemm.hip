@@ -705,10 +705,11 @@ hipError_t launch_to_bf16_pairs(const double* x, long count, unsigned* out, hipS
 namespace {
 constexpr int kOnsiteRows = 64;  // projector rows of one workgroup
 
-// Onsite products straight from the projection's split-K partials: P (the partials
-// of a column summed in split order) lives in LDS only, then per atom W(:, 0:m) =
-// D P and W(:, m:2m) = Q P, or with `shift` W(:, 0:m) = (D - shift_j Q) P in one
-// pass. Workgroup (g, j): atoms [group_atom[g], group_atom[g + 1]) (at most
+// Onsite products straight from the projection's split-K partials: P (the quarters of
+// a column's partials each summed in split order, then the four sums in theirs, which
+// rounds unlike k_splitk_reduce's single chain) lives in LDS only, then per atom
+// W(:, 0:m) = D P and W(:, m:2m) = Q P, or with `shift` W(:, 0:m) = (D - shift_j Q) P in
+// one pass. Workgroup (g, j): atoms [group_atom[g], group_atom[g + 1]) (at most
 // kOnsiteRows rows, or one larger atom), column j. Bound: latency of the partials
 // (each read once). FP64 keeps the compensated scalar order of k_atom_blocks_comp.
 template <typename T>
@@ -833,6 +834,16 @@ std::vector<int> onsite_groups(const std::vector<int>& atom_rows) {
   }
   first.push_back(int(atom_rows.size()));
   return first;
+}
+
+int onsite_group_rows(const std::vector<int>& atom_rows, const std::vector<int>& groups) {
+  int most = 0;
+  for (std::size_t g = 0; g + 1 < groups.size(); ++g) {
+    int rows = 0;
+    for (int a = groups[g]; a < groups[g + 1]; ++a) rows += atom_rows[std::size_t(a)];
+    most = std::max(most, rows);
+  }
+  return most;
 }
 
 hipError_t launch_onsite_partials(Precision prec, int np, int columns, int splits, const double* partial,

@@ -74,6 +74,8 @@ hipError_t launch_atom_blocks(Precision prec, int np, int columns, int atoms, co
 // most kOnsiteGroupRows.
 constexpr int kOnsiteGroupRows = 1024;
 std::vector<int> onsite_groups(const std::vector<int>& atom_rows);
+// rows of the largest group
+int onsite_group_rows(const std::vector<int>& atom_rows, const std::vector<int>& groups);
 hipError_t launch_onsite_partials(Precision prec, int np, int columns, int splits, const double* partial,
                                   const int* group_atom, int groups, int group_rows, const int* atom_offset,
                                   const int* atom_rows, const long* block_offset, const double* dblk,

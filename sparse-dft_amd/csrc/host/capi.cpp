@@ -365,7 +365,6 @@ int sdft_hip_paw_pair(sdft_hip_context* ctx, uint64_t identity, size_t npw, size
     cx.zgemm(prec, 0, 0, M, N, K, 1.0, P.b.p, M, P.in.p, K, P.p.p, M, nullptr, 0, 0.0);
     cx.zgemm(prec, 0, 0, M, N, M, 1.0, P.d.p, M, P.p.p, M, P.dq.p, M, nullptr, 0, 0.0);
     cx.zgemm(prec, 0, 0, M, N, M, 1.0, P.q.p, M, P.p.p, M, P.dq.p + 2 * M * N, M, nullptr, 0, 0.0);
-    // one back-projection GEMM over [DP | QP] (2 columns blocks)
     double* hs = P.h.p;
     cx.zgemm(prec, 1, 0, K, N, M, 1.0, P.b.p, M, P.dq.p, M, hs, K, nullptr, 0, 0.0);
     cx.zgemm(prec, 1, 0, K, N, M, 1.0, P.b.p, M, P.dq.p + 2 * M * N, M, P.s.p, K, nullptr, 0, 0.0);
@@ -915,40 +914,64 @@ int sdft_hip_tridiagonal_eigen(sdft_hip_context* ctx, size_t n, const double* d,
   });
 }
 
+namespace {
+// W = [D_a P_a | Q_a P_a] of P's partial sums by the kernel that an application takes;
+// `partials_only`: not by the one for atoms too large to be summed there.
+void onsite_products(sdft_hip_context* ctx, std::size_t atoms, const long* rows, const double* d, const double* q,
+                     std::size_t splits, const double* p, std::size_t columns, double* w, int precision,
+                     bool partials_only) {
+  if (!ctx || !atoms || !rows || !d || !q || !p || !w || !columns || !splits)
+    throw std::invalid_argument("HIP: invalid onsite block arguments");
+  auto& cx = ctx->impl;
+  hipStream_t s = cx.stream();
+  std::vector<int> offs, rws;
+  std::vector<long> boffs;
+  std::size_t np = 0, bo = 0;
+  for (std::size_t a = 0; a < atoms; ++a) {
+    if (rows[a] <= 0) throw std::invalid_argument("HIP: invalid onsite block size");
+    offs.push_back(int(np));
+    rws.push_back(int(rows[a]));
+    boffs.push_back(long(bo));
+    np += std::size_t(rows[a]);
+    bo += std::size_t(rows[a]) * std::size_t(rows[a]);
+  }
+  check_int_range({np, columns, splits});
+  const std::vector<int> first = sdft_hip::onsite_groups(rws);
+  const int groups = int(first.size()) - 1, group_rows = sdft_hip::onsite_group_rows(rws, first);
+  const bool direct = group_rows <= sdft_hip::kOnsiteGroupRows && columns <= 65535;
+  if (partials_only && !direct) throw std::invalid_argument("HIP: onsite blocks beyond the partial sums' kernel");
+  DevBuf<int> doff, drow, dfirst;
+  DevBuf<long> dbo;
+  DevBuf<double> dd, dq, dp, dw;
+  doff.upload(offs.data(), offs.size(), s);
+  drow.upload(rws.data(), rws.size(), s);
+  dfirst.upload(first.data(), first.size(), s);
+  dbo.upload(boffs.data(), boffs.size(), s);
+  dd.upload(d, 2 * bo, s);
+  dq.upload(q, 2 * bo, s);
+  dp.upload(p, 2 * np * columns * splits, s);
+  dw.reserve(4 * np * columns);
+  if (direct)
+    check(sdft_hip::launch_onsite_partials(to_precision(precision), int(np), int(columns), int(splits), dp.p, dfirst.p,
+                                           groups, group_rows, doff.p, drow.p, dbo.p, dd.p, dq.p, nullptr, dw.p, 3, s),
+          "onsite blocks");
+  else
+    check(sdft_hip::launch_atom_blocks(to_precision(precision), int(np), int(columns), int(atoms), doff.p, drow.p,
+                                       dbo.p, dd.p, dq.p, dp.p, long(np), dw.p, long(np), 3, s),
+          "onsite blocks");
+  check(hipMemcpyAsync(w, dw.p, 32 * np * columns, hipMemcpyDeviceToHost, s), "copy");
+  cx.sync();
+}
+}  // namespace
+
 int sdft_hip_onsite_blocks(sdft_hip_context* ctx, size_t atoms, const long* rows, const double* d, const double* q,
                            const double* p, size_t columns, double* w, int precision) {
-  return guarded([&] {
-    if (!ctx || !atoms || !rows || !d || !q || !p || !w || !columns)
-      throw std::invalid_argument("HIP: invalid onsite block arguments");
-    auto& cx = ctx->impl;
-    hipStream_t s = cx.stream();
-    std::vector<int> offs, rws;
-    std::vector<long> boffs;
-    std::size_t np = 0, bo = 0;
-    for (std::size_t a = 0; a < atoms; ++a) {
-      if (rows[a] <= 0) throw std::invalid_argument("HIP: invalid onsite block size");
-      offs.push_back(int(np));
-      rws.push_back(int(rows[a]));
-      boffs.push_back(long(bo));
-      np += std::size_t(rows[a]);
-      bo += std::size_t(rows[a]) * std::size_t(rows[a]);
-    }
-    DevBuf<int> doff, drow;
-    DevBuf<long> dbo;
-    DevBuf<double> dd, dq, dp, dw;
-    doff.upload(offs.data(), offs.size(), s);
-    drow.upload(rws.data(), rws.size(), s);
-    dbo.upload(boffs.data(), boffs.size(), s);
-    dd.upload(d, 2 * bo, s);
-    dq.upload(q, 2 * bo, s);
-    dp.upload(p, 2 * np * columns, s);
-    dw.reserve(4 * np * columns);
-    check(sdft_hip::launch_atom_blocks(to_precision(precision), int(np), int(columns), int(atoms), doff.p, drow.p, dbo.p,
-                                       dd.p, dq.p, dp.p, long(np), dw.p, long(np), 3, s),
-          "onsite blocks");
-    check(hipMemcpyAsync(w, dw.p, 32 * np * columns, hipMemcpyDeviceToHost, s), "copy");
-    cx.sync();
-  });
+  return guarded([&] { onsite_products(ctx, atoms, rows, d, q, 1, p, columns, w, precision, false); });
+}
+
+int sdft_hip_onsite_partials(sdft_hip_context* ctx, size_t atoms, const long* rows, const double* d, const double* q,
+                             size_t splits, const double* partials, size_t columns, double* w, int precision) {
+  return guarded([&] { onsite_products(ctx, atoms, rows, d, q, splits, partials, columns, w, precision, true); });
 }
 
 }  // extern "C"

@@ -601,12 +601,7 @@ void DeviceOperator::set_chunk() {
 void DeviceOperator::upload_onsite_groups() {
   const std::vector<int> first = onsite_groups(atom_rows_host_);
   onsite_groups_ = int(first.size()) - 1;
-  onsite_group_rows_ = 0;
-  for (int g = 0; g < onsite_groups_; ++g) {
-    int rows = 0;
-    for (int a = first[g]; a < first[g + 1]; ++a) rows += atom_rows_host_[a];
-    onsite_group_rows_ = std::max(onsite_group_rows_, rows);
-  }
+  onsite_group_rows_ = onsite_group_rows(atom_rows_host_, first);
   onsite_group_.upload(first.data(), first.size(), ctx_.stream());
   ctx_.sync();  // `first` ends here
 }

@@ -374,6 +374,19 @@ class Context:
                                             ct.c_size_t(cols), _p(w), ct.c_int(precision)))
         return w
 
+    def onsite_partials(self, rows, d_blocks, q_blocks, partials, precision=0):
+        """onsite_blocks of the sum of `partials` (splits x projectors x columns)."""
+        rows = np.ascontiguousarray(rows, dtype=np.int64)
+        d = np.ascontiguousarray(np.concatenate([np.asfortranarray(b).ravel(order="F") for b in d_blocks]))
+        q = np.ascontiguousarray(np.concatenate([np.asfortranarray(b).ravel(order="F") for b in q_blocks]))
+        splits, npj, cols = partials.shape
+        p = np.ascontiguousarray(np.swapaxes(partials, 1, 2), dtype=np.complex128)
+        w = np.zeros((npj, 2 * cols), dtype=np.complex128, order="F")
+        _check(lib().sdft_hip_onsite_partials(self.handle, ct.c_size_t(len(rows)), _p(rows, _lp), _p(d), _p(q),
+                                              ct.c_size_t(splits), _p(p), ct.c_size_t(cols), _p(w),
+                                              ct.c_int(precision)))
+        return w
+
 
 def pack_problem(prob):
     """The operator description of a Problem as contiguous arrays (the layout

@@ -12,6 +12,7 @@
 
 #include "gemm.hpp"
 #include "gemm_plan.hpp"
+#include "lds_barrier.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -130,15 +131,6 @@ struct Slab {
   }
 };
 
-// Workgroup barrier over LDS data only: the next slab's loads stay in flight
-// (__syncthreads waits for them). 0xC07F: lgkmcnt(0), the other counters free.
-__device__ __forceinline__ void slab_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-}
-
 // One TBM x TBN output tile per 256-thread workgroup (2 x 2 waves), K range
 // [k0, k1) of this split. Each wave computes (TBM/2) x (TBN/2) as 16 x 16 blocks:
 // per 4-deep K step one LDS read an operand block (re and im together) and three
@@ -181,7 +173,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
   sb.load(pb, tid, k1 - k0);
   sa.template store<ADJ_A>(lds_a[0], tid);
   sb.template store<ADJ_B>(lds_b[0], tid);
-  slab_barrier();
+  lds_barrier();
   int buffer = 0;
   for (int kb = k0; kb < k1; kb += BK) {
     const bool more = kb + BK < k1;
@@ -218,7 +210,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
       buffer ^= 1;
       sa.template store<ADJ_A>(lds_a[buffer], tid);
       sb.template store<ADJ_B>(lds_b[buffer], tid);
-      slab_barrier();
+      lds_barrier();
     }
   }
   // Accumulator layout of each 16x16 block (columns of C^T = rows of C along the

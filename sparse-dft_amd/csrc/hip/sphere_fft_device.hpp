@@ -5,6 +5,7 @@
 #include "fft_device.hpp"
 #include "fft_dispatch.hpp"
 #include "fft_lengths.hpp"
+#include "lds_barrier.hpp"
 
 namespace sdft_hip {
 
@@ -32,15 +33,6 @@ constexpr bool keeps(int n) {
 __device__ __forceinline__ void wave_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
-}
-
-// Workgroup barrier over LDS data only: global loads in flight stay in flight
-// (__syncthreads waits for them). 0xC07F: lgkmcnt(0), the other counters free.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
 // A buffer accessed by 32-bit byte offsets: one past the end (kOutside, or that

@@ -48,3 +48,25 @@ def test_far_leading_dimension(hip_ctx, ops):
     c = np.zeros(m * n, dtype=np.complex128)
     hip_ctx.zgemm_strided(ops[0], 0, m, n, k, a.ravel(order="F"), ld, b.ravel(order="F"), ld, c, m)
     assert np.abs(c.reshape((m, n), order="F") - left @ b[:k, :n]).max() <= 1e-13
+
+
+# one operand past that reach: planned as 64 x 32 tiles in 46 splits whose last is ragged
+# (then run as 32 x 32 with the same K ranges), with the other operand normal and
+# adjoint; several tiles and slabs along the far operand's columns; an adjoint B
+@pytest.mark.parametrize("far,ops,mnk", [("a", (1, 0), (5, 512, 12301)), ("a", (1, 1), (5, 512, 12301)),
+                                         ("a", (0, 0), (70, 40, 17)), ("b", (0, 1), (40, 70, 17)),
+                                         ("b", (1, 0), (70, 5, 6001))])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_one_far_operand(hip_ctx, far, ops, mnk, precision):
+    m, n, k = mnk
+    rng = np.random.default_rng(5)
+    shape_a, shape_b = (m, k) if not ops[0] else (k, m), (k, n) if not ops[1] else (n, k)
+    a = _operand(rng, *shape_a, ld=(1 << 20) + 3 if far == "a" else shape_a[0])
+    b = _operand(rng, *shape_b, ld=(1 << 20) + 5 if far == "b" else shape_b[0])
+    left = a[:m, :k] if not ops[0] else a[:k, :m].conj().T
+    right = b[:k, :n] if not ops[1] else b[:n, :k].conj().T
+    c = np.zeros(m * n, dtype=np.complex128)
+    hip_ctx.zgemm_strided(*ops, m, n, k, a.ravel(order="F"), a.shape[0], b.ravel(order="F"), b.shape[0], c, m,
+                          precision=precision)
+    eps = 2.0 ** -53 if precision == 0 else 2.0 ** -24
+    assert np.abs(c.reshape((m, n), order="F") - left @ right).max() <= 32 * eps * k ** 0.5 * np.log2(k + 1) + 32 * eps

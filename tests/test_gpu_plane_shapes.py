@@ -50,3 +50,28 @@ def test_local_hamiltonian_grid_and_sphere(hip_ctx, shape, sphere, precision):
     # log2 of the grid, on the scale of the largest entry
     eps = 2.0 ** -53 if precision == 0 else 2.0 ** -24
     assert np.abs(got - ref).max() <= 64 * eps * np.abs(ref).max()
+
+
+# 96 x 96: with every line touched, a plane and its waves' buffers pass the LDS of a
+# workgroup in FP64 (98 rows of 97 and 4 x 480 values of 16 bytes: 183 kB) and the
+# in-place kernel takes over
+@pytest.mark.parametrize("sphere", sorted(SPHERES))
+@pytest.mark.parametrize("precision", [0, 1])
+def test_local_hamiltonian_plane_beyond_the_lds(hip_ctx, sphere, precision):
+    indices, kinetic, potential, x, ref = _case((96, 96, 3), sphere, 2, 12)
+    got = hip_ctx.local_hamiltonian((96, 96, 3), indices, kinetic, potential, x, precision=precision)
+    eps = 2.0 ** -53 if precision == 0 else 2.0 ** -24
+    assert np.abs(got - ref).max() <= 64 * eps * np.abs(ref).max()
+
+
+# z-lines with a register DFT above 10 (5 x 15, 8 x 12, 9 x 14, 8 x 16), by one-wave
+# workgroups and, from 512 of four waves on, by those
+@pytest.mark.parametrize("shape", [(4, 5, 75), (12, 10, 96), (3, 4, 126), (6, 8, 128)])
+@pytest.mark.parametrize("sphere", sorted(SPHERES))
+@pytest.mark.parametrize("columns", [3, 400])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_local_hamiltonian_long_lines(hip_ctx, shape, sphere, columns, precision):
+    indices, kinetic, potential, x, ref = _case(shape, sphere, columns, 13)
+    got = hip_ctx.local_hamiltonian(shape, indices, kinetic, potential, x, precision=precision)
+    eps = 2.0 ** -53 if precision == 0 else 2.0 ** -24
+    assert np.abs(got - ref).max() <= 64 * eps * np.abs(ref).max()

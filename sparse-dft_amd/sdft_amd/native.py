@@ -343,7 +343,8 @@ class Context:
         kin = np.ascontiguousarray(kinetic, dtype=np.float64)
         pot = np.ascontiguousarray(potential, dtype=np.float64)
         x = np.asfortranarray(x, dtype=np.complex128)
-        out = np.empty_like(x, order="F")
+        # the library writes len(idx) values a column, all of `out` where x is as long
+        out = (np.empty_like if len(x) == len(idx) else np.zeros_like)(x, order="F")
         _check(lib().sdft_hip_local_hamiltonian(self.handle, _p(shp, _ip), _p(idx, _u64p), ct.c_size_t(len(idx)),
                                                 _p(kin), _p(pot), _p(x), ct.c_size_t(x.shape[1]), _p(out),
                                                 ct.c_uint64(operator_identity), ct.c_int(precision)))

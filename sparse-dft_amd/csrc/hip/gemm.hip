@@ -139,8 +139,8 @@ struct Slab {
 // with one barrier a slab. The MFMA takes the operands exchanged (C^T = B^T A^T),
 // so that a lane's results lie along M: stores of 256 contiguous bytes.
 // Bound: FP64 by the MFMA rate at the clock that FP64 MFMA load leaves (near
-// 2.0 GHz: 78 % of the CU's cycles issue MFMAs); FP32 70 % of them. WAVES: at
-// least that many waves per SIMD.
+// 2.0 GHz; the matrix cores are busy in 72 to 77 % of the cycles of the 64-atom
+// products, 67 % in FP32). WAVES: at least that many waves per SIMD.
 template <typename T, typename TA, typename TB, bool ADJ_A, bool ADJ_B, int TBM, int TBN, bool FAR, int WAVES>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_zgemm(
     int M, int N, int K, const TA* __restrict__ A, long lda, const TB* __restrict__ B, long ldb, GemmOutput first,

@@ -229,7 +229,7 @@ __device__ __forceinline__ void y_out(cx<T>* rows, const PlaneRows& pr, const Bu
   }
 }
 
-// grid (n2 z slots, columns). Bound: vector issue in FP32 (95 % of the cycles),
+// grid (n2 z slots, columns). Bound: vector issue in FP32 (96 % of the cycles),
 // latency in FP64 (half of them; the registers hold three waves a SIMD, the LDS two of
 // them at 72 x 72); HBM carries only the sticks. Measured alone, in-place plane kernel ->
 // this one: 160 columns of 72^3 627 -> 308 us FP64 and 301 -> 163 us FP32, 96 columns of

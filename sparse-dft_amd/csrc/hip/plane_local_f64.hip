@@ -7,8 +7,12 @@ template bool plan_plane_local<double>(const GridPlanDev&, PlaneLocalPlan&);
 template hipError_t launch_plane_local<double>(const GridPlanDev&, const PlaneLocalPlan&, const void*, void*, long,
                                               hipStream_t);
 
-// Loads this file's code object on the calling thread (see module_prime.hpp).
+// Loads this file's code object on the calling thread (see module_prime.hpp) and asks
+// what the launch rule will want to know, so that no application does.
 hipError_t prime_module_plane_local_f64() {
+  (void)plane_local::register_waves<double, true, false>();
+  (void)plane_local::register_waves<double, false, true>();
+  (void)plane_local::register_waves<double, false, false>();
   hipFuncAttributes a{};
   return hipFuncGetAttributes(&a, reinterpret_cast<const void*>(plane_local::k_plane_local<double, false, true>));
 }
